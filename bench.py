@@ -48,6 +48,10 @@ STAGES = ("route", "permute", "gemm1_swiglu", "gemm2", "combine")
 GEMM1_STREAM_MAX_ROWS = 4
 GEMM1_BIG_ROWS = 16
 GEMM2_TILE_MAX_ROWS = 7
+# ... and of justgoal_amd/csrc/moe_wide.hip (kBigTileRows, kMinRounds), on 256 CUs
+GEMM2_BIG_TILE_ROWS = 64
+GEMM2_WIDE_MIN_ROUNDS = 5
+CUS = 256
 
 
 def log(msg):
@@ -261,10 +265,15 @@ def gemm1_kernel_name(cfg):
 
 
 def gemm2_kernel_name(cfg):
-    """GEMM2: LDS-tiled up to GEMM2_TILE_MAX_ROWS expected pairs per expert, large tiles above
-    (every bench geometry has I >= 384, which the LDS-tiled kernel needs)."""
-    return ("gemm2_tile_kernel" if _rows_hint(cfg) <= GEMM2_TILE_MAX_ROWS
-            else "gemm2_big_kernel")
+    """GEMM2: LDS-tiled up to GEMM2_TILE_MAX_ROWS expected pairs per expert; above, 256-column
+    tiles from GEMM2_BIG_TILE_ROWS, or where the experts' tiles fill the chip
+    GEMM2_WIDE_MIN_ROUNDS times; else large tiles (every bench geometry has I >= 384)."""
+    rows, g = _rows_hint(cfg), cfg.geom
+    if rows <= GEMM2_TILE_MAX_ROWS:
+        return "gemm2_tile_kernel"
+    tiles = g.local_experts * -(-g.hidden // 256)
+    wide = rows >= GEMM2_BIG_TILE_ROWS or tiles >= GEMM2_WIDE_MIN_ROUNDS * CUS
+    return "gemm2_wide_kernel" if wide else "gemm2_big_kernel"
 
 
 def load_traffic(stage, name):

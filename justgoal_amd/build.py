@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB_NAME = "libjustgoal_moe.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
-SOURCES = ["moe_api.hip", "moe_routing.hip", "moe_gemm.hip", "moe_stream.hip", "moe_tile.hip", "moe_big.hip", "moe_quant.hip"]
+SOURCES = ["moe_api.hip", "moe_routing.hip", "moe_gemm.hip", "moe_stream.hip", "moe_tile.hip", "moe_big.hip", "moe_wide.hip", "moe_quant.hip"]
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -1,18 +1,17 @@
-// Large-tile grouped GEMMs for longer per-expert segments (GEMM1 from 16 expected pairs per
-// expert, GEMM2 from 8; GEMM2's padding-row skip keeps part-filled tiles cheap).
+// Large-tile grouped GEMMs with a producer wave: GEMM1 from 16 expected pairs per expert, GEMM2
+// from 8 to 63 where 256-column tiles (moe_wide.hip) would leave the last round too empty.
 //
-// A workgroup (one per CU) computes a 128-row x 128-column output tile of one expert with eight
-// compute waves (GEMM1: 2x4 grid, wave tile 64 rows x 32 C columns; GEMM2: 4x2, 32 rows x 64 H
-// columns) and one producer wave. Both operands reach LDS by DMA into a 3-slot ring, so every
-// weight K-block is fetched once per 128 rows and every activation K-block once per 128
-// columns. The same kernels are instantiated with 64-row tiles for shorter segments (2x4 waves
-// of 32 x 32; GEMM2 then has room for a 4-slot ring) and, for GEMM1 from 64 to 159 expected
-// rows, with four compute waves of 64 x 64; the launchers below pick the form:
+// A workgroup (one per CU) computes a tile of one expert with eight compute waves (or four) and one
+// producer wave. GEMM1: 128 rows x 128 C columns (2x4 waves of 64 rows x 32 C columns, or, from 64
+// to 159 expected rows, 2x2 of 64 x 64; 64-row tiles, 2x4 waves of 32 x 32, below 64). GEMM2: 64
+// rows x 128 H columns (2x4 waves of 32 x 32). Both operands reach LDS by DMA into a 3-slot
+// (GEMM2: 4-slot) ring, so every weight K-block is fetched once per tile height and every activation
+// K-block once per 128 columns:
 //
 // * GEMM1: 128 rows of fp8 hidden states (gathered through the pair -> token list) plus their
 //   activation scales, and 128 columns of C, i.e. 128 X1 rows and 128 X2 rows of W13. The
 //   epilogue applies SwiGLU and stores bf16 C.
-// * GEMM2: 128 rows of bf16 C and 128 rows of W2; the epilogue scales by the pair's routing
+// * GEMM2: 64 rows of bf16 C and 128 rows of W2; the epilogue scales by the pair's routing
 //   weight and stores bf16 rows at the pair's destination (the token's output row for its first
 //   local pair, else one of its partial rows for the combine).
 //
@@ -32,45 +31,6 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kWBlk = 16 * kBlock;  // 16 rows x 128 bytes
-
-// A buffer offset past every buffer these kernels address (all are < 2 GiB; the launchers check).
-constexpr uint32_t kOutOfRange = 0x7ffffff0u;
-
-// Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs on XCD b % 8), and the
-// persistent loop hands workgroup b the items b, b + grid, ... (grid a multiple of 8). This
-// bijection on [0, items) gives XCD x a contiguous run of the logical item list instead of
-// every 8th item, so consecutive logical items meet in the same L2.
-__device__ __forceinline__ int xcd_item(int i, int items) {
-  const int x = i & 7, q = items >> 3, r = items & 7;
-  return x * q + (x < r ? x : r) + (i >> 3);
-}
-
-// Work item -> (expert, first row m0 of its M-tile, N-tile nt). sched bit 0: XCD-contiguous
-// physical order (xcd_item); sched >> 1 = GM: 0 = tile-major logical order (the N-tiles of one
-// M-tile consecutive), else each expert's M-tiles in bands of GM with the band's items
-// N-tile-major (GM M-tiles of one N-tile consecutive).
-template <int BM>
-__device__ __forceinline__ int map_item(const TileMapLds& tml, int item, int items, int NNT,
-                                        int E_l, int sched, int& m0, int& cnt, int& seg,
-                                        int& nt) {
-  item = uniform((sched & 1) ? xcd_item(item, items) : item);
-  const int tile = item / NNT;
-  const int e = uniform(tml.template find<BM>(tile, E_l, m0, cnt, seg));
-  nt = item - tile * NNT;
-  const int GM = sched >> 1;
-  if (GM > 0) {
-    const int first = tile - uniform(m0) / BM;  // the expert's first tile slot
-    const int me = (uniform(cnt) + BM - 1) / BM;
-    const int local = item - first * NNT;
-    const int band = local / (GM * NNT);
-    const int rows = min(GM, me - band * GM);
-    const int idx = local - band * GM * NNT;
-    nt = idx / rows;
-    m0 = (band * GM + idx % rows) * BM;
-  }
-  nt = uniform(nt);
-  return e;
-}
 
 constexpr int vm_depth(int n) { return n > 63 ? 63 : n < 0 ? 0 : n; }
 
@@ -786,8 +746,7 @@ __global__ __launch_bounds__((WM * WN + 1) * kWave) void gemm2_big_kernel(
 // up to 8 M-tiles and activation rows across 4 N-tiles. For GEMM1 it fetches fewer bytes than
 // the tile-major round-robin order (T=4096: 0.89 against 1.19 GB, algorithmic 0.80; T=16384
 // skewed: 6.07 against 7.96 GB) and made the Qwen3-style T=1024 batch's GEMM1 364 -> 327 us.
-// GEMM2 keeps the tile-major round-robin order: every variant tried (XCD-contiguous, bands of
-// 2-16) was 1-5% slower there.
+// GEMM2's 64-row tiles keep the tile-major round-robin order.
 constexpr int kSchedGemm1 = 1 | (8 << 1);
 constexpr int kSchedGemm2 = 0;
 // Tile-major round-robin puts item i on XCD i % 8. When an expert has a multiple of 8 N-tiles,
@@ -835,29 +794,19 @@ constexpr int kB1ShortMs = 2;
 // 382.3 -> 371.0. From 160 rows, where GEMM1 turns MFMA-bound, the 8-wave form, whose two waves
 // per SIMD overlap one's MFMAs with the other's scale FMAs, is ahead: T=5120 235.2 against
 // 240.9, T=6144 248.7 against 256.6, T=8192 334.5 against 341.3, T=16384 skewed 1922 against
-// 2006. The same 2 x 2 layout measured within 1% for the 64-row tiles of both GEMMs, and 4-8%
-// slower for GEMM2's 128-row tiles (2 x 2, or 4 x 1 waves of 32 x 128) at T=2048-16384.
+// 2006. The same 2 x 2 layout measured within 1% for the 64-row tiles of both GEMMs.
 constexpr int kB1EightWaveRows = 160;
 constexpr int kB1WideNs = 4;
 constexpr int kB1WideWm = 2;
 constexpr int kB1WideWn = 2;
+// GEMM2 for 8..63 expected rows per expert, unless the experts' 256-column tiles fill the chip
+// often enough (moe_wide.hip): 64-row x 128-column tiles (2 x 4 waves of 32 x 32) in a 4-slot
+// ring (146 KB of LDS). A 3-slot ring was 0.4-1.5% behind the 4-slot one everywhere.
 constexpr int kB2Ms = 2;
-constexpr int kB2Ns = 4;
-constexpr int kB2Wm = 4;
-constexpr int kB2Wn = 2;
-constexpr int kB2D = 3;
-// GEMM2 for 8..63 expected rows per expert: 64-row tiles (2 x 4 waves of 32 x 32, NS = 2) in a
-// 4-slot ring (146 KB of LDS). Against the 128-row tiles, whole call, two weight sets in
-// rotation, results bit-identical: DS-V3 T=768 252.1 -> 236.6 us, T=1024 260.6 -> 249.8,
-// T=1280 283.0 -> 275.4, T=1536 310.0 -> 306.9, T=1792 344.1 -> 339.9; Qwen3-style T=512 503.3 ->
-// 486.0, T=640 515.0 -> 504.0, T=768 541.2 -> 534.4. From 64 rows the 128-row tiles stay ahead
-// (DS-V3 T=2048 299.8 against 304.6, Qwen3-style T=1024 554.0 against 568.4). A 3-slot ring
-// was 0.4-1.5% behind the 4-slot one everywhere.
-constexpr int kB2TallRows = 64;
-constexpr int kB2ShortWm = 2;
-constexpr int kB2ShortWn = 4;
-constexpr int kB2ShortNs = 2;
-constexpr int kB2ShortD = 4;
+constexpr int kB2Ns = 2;
+constexpr int kB2Wm = 2;
+constexpr int kB2Wn = 4;
+constexpr int kB2D = 4;
 
 template <int MS, int NS, int D, int WM, int WN>
 static hipError_t launch_gemm1_big_t(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,
@@ -905,13 +854,8 @@ static hipError_t launch_gemm2_big_t(const uint16_t* C, const uint8_t* w2, const
 
 hipError_t launch_gemm2_big(const uint16_t* C, const uint8_t* w2, const float* s2,
                             const int32_t* counts, const int32_t* offsets, const float* sorted_w,
-                            Gemm2Out dst, int H, int I, int E_l, int max_pairs, int rows_hint,
+                            Gemm2Out dst, int H, int I, int E_l, int max_pairs,
                             hipStream_t stream) {
-  if (rows_hint < kB2TallRows) {
-    const hipError_t e = launch_gemm2_big_t<kB2Ms, kB2ShortNs, kB2ShortD, kB2ShortWm, kB2ShortWn>(
-        C, w2, s2, counts, offsets, sorted_w, dst, H, I, E_l, max_pairs, stream);
-    if (e != hipErrorNotSupported) return e;  // I = 256: the 4-slot ring needs 3 K blocks
-  }
   return launch_gemm2_big_t<kB2Ms, kB2Ns, kB2D, kB2Wm, kB2Wn>(C, w2, s2, counts, offsets,
                                                               sorted_w, dst, H, I, E_l,
                                                               max_pairs, stream);

@@ -386,6 +386,45 @@ struct TileMapLds {
   }
 };
 
+// A buffer offset past every buffer these kernels address (all are < 2 GiB; the launchers check).
+constexpr uint32_t kOutOfRange = 0x7ffffff0u;
+
+// Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs on XCD b % 8), and the
+// persistent loop hands workgroup b the items b, b + grid, ... (grid a multiple of 8). This
+// bijection on [0, items) gives XCD x a contiguous run of the logical item list instead of
+// every 8th item, so consecutive logical items meet in the same L2.
+__device__ __forceinline__ int xcd_item(int i, int items) {
+  const int x = i & 7, q = items >> 3, r = items & 7;
+  return x * q + (x < r ? x : r) + (i >> 3);
+}
+
+// Work item -> (expert, first row m0 of its M-tile, N-tile nt). sched bit 0: XCD-contiguous
+// physical order (xcd_item); sched >> 1 = GM: 0 = tile-major logical order (the N-tiles of one
+// M-tile consecutive), else each expert's M-tiles in bands of GM with the band's items
+// N-tile-major (GM M-tiles of one N-tile consecutive).
+template <int BM>
+__device__ __forceinline__ int map_item(const TileMapLds& tml, int item, int items, int NNT,
+                                        int E_l, int sched, int& m0, int& cnt, int& seg,
+                                        int& nt) {
+  item = uniform((sched & 1) ? xcd_item(item, items) : item);
+  const int tile = item / NNT;
+  const int e = uniform(tml.template find<BM>(tile, E_l, m0, cnt, seg));
+  nt = item - tile * NNT;
+  const int GM = sched >> 1;
+  if (GM > 0) {
+    const int first = tile - uniform(m0) / BM;  // the expert's first tile slot
+    const int me = (uniform(cnt) + BM - 1) / BM;
+    const int local = item - first * NNT;
+    const int band = local / (GM * NNT);
+    const int rows = min(GM, me - band * GM);
+    const int idx = local - band * GM * NNT;
+    nt = idx / rows;
+    m0 = (band * GM + idx % rows) * BM;
+  }
+  nt = uniform(nt);
+  return e;
+}
+
 // Total M-tiles over all experts: sum of ceil(count / bm). Wave-uniform; every lane must call.
 __device__ __forceinline__ int count_m_tiles(const int32_t* __restrict__ counts, int n_experts,
                                              int bm) {

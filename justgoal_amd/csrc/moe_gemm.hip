@@ -1,13 +1,15 @@
 // Kernel selection for the two expert GEMMs, and the weighted combine.
 //
 // The GEMMs themselves live in moe_stream.hip (weight streaming, a few pairs per expert),
-// moe_tile.hip (LDS-tiled GEMM1) and moe_big.hip (large tiles). Their arithmetic is the same:
+// moe_tile.hip (LDS-tiled), moe_big.hip (large tiles) and moe_wide.hip (GEMM2's 256-column tiles).
+// Their arithmetic is the same:
 // GEMM1 runs one v_mfma_f32_16x16x128_f8f6f4 per 128-wide K scale block and adds its fp32 result
 // times hs_scale[kb, token] * s13[e, n/128, kb] to the accumulator
 // (goal_full_shape/opus-4.8/moe_fp8_fwd/MOEDIR/main.py:125-132), then applies SwiGLU into bf16 C
 // (not requantised to fp8 as the reference solutions do at main.py:151-156); GEMM2 converts the
 // W2 e4m3 bytes to bf16 exactly, runs four v_mfma_f32_16x16x32_bf16 per K block (lane group
-// g = lane>>4 carries K = 32g + 8c .. +8 for instruction c, the same map on both operands), scales
+// g = lane>>4 carries K = 32g + 8c .. +8 for instruction c, the same map on both operands; the
+// wide kernel eight v_mfma_f32_32x32x16_bf16), scales
 // by s2[e, h/128, kb] and stores bf16 rows times the pair's routing weight at the pair's
 // destination row (out for a token's first local pair, else a partial row for combine_kernel).
 //
@@ -70,9 +72,10 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(
 // over DS-V3 T = 16..16384 and Qwen3-style T = 32..1024. GEMM1 streams weights up to 4 expected
 // rows, uses the LDS-tiled kernels up to 15 and the large-tile kernel from 16 (64-row tiles up to
 // 63, 128-row tiles from 64; moe_big.hip has the measurements). GEMM2 uses the LDS-tiled
-// kernel up to 7 expected rows (16-row tiles at <= 1, 32-row tiles above) and the large-tile
-// kernel from 8 (64-row tiles up to 63, 128-row tiles from 64); the streaming GEMM2 remains the
-// fallback for shapes the tiled kernel does not take.
+// kernel up to 7 expected rows (16-row tiles at <= 1, 32-row tiles above), from 8 to 63 the
+// large-tile kernel's 64 x 128 tiles or, over many experts, the wide kernel, and from 64 the wide
+// kernel's 128 x 256 tiles (moe_wide.hip has the measurements); the streaming GEMM2 remains the
+// fallback for shapes these do not take (I < 256, and up to 7 rows I < 384).
 // The streaming kernels' 16-row items re-stream an expert's weights once per 16 rows, so they
 // only win while segments are that short; the tiled GEMM2 shares one staged C tile among four
 // waves and streams each weight block once per 32 rows. Against streaming up to 4 rows and large
@@ -127,8 +130,11 @@ hipError_t launch_gemm2(const uint16_t* C, const uint8_t* w2, const float* s2,
     if (t != hipErrorNotSupported) return t;
   }
   if (rows_hint > kG2TileMaxRows) {
+    const hipError_t v = launch_gemm2_wide(C, w2, s2, counts, offsets, sorted_w, dst, H, I, E_l,
+                                           max_pairs, rows_hint, stream);
+    if (v != hipErrorNotSupported) return v;
     const hipError_t b = launch_gemm2_big(C, w2, s2, counts, offsets, sorted_w, dst, H, I, E_l,
-                                          max_pairs, rows_hint, stream);
+                                          max_pairs, stream);
     if (b != hipErrorNotSupported) return b;
   }
   return launch_gemm2_stream(C, w2, s2, counts, offsets, sorted_w, dst, H, I, E_l, max_pairs,

@@ -72,6 +72,19 @@ def test_kernel_family_thresholds_match_the_library_source():
     assert g2names["ds_t1024"] == "gemm2_big_kernel"
 
 
+def test_gemm2_wide_rule_matches_the_library_source():
+    import re
+    from justgoal_amd import inputs as jin
+    src = open(os.path.join(ROOT, "justgoal_amd", "csrc", "moe_wide.hip")).read()
+    rows = int(re.search(r"constexpr int kBigTileRows = (\d+);", src).group(1))
+    rounds = int(re.search(r"constexpr int kMinRounds = (\d+);", src).group(1))
+    assert (bench.GEMM2_BIG_TILE_ROWS, bench.GEMM2_WIDE_MIN_ROUNDS) == (rows, rounds)
+    names = {n: bench.gemm2_kernel_name(c) for n, c in jin.CONFIGS.items()}
+    assert names["ds_t2048"] == names["ds_t16384_skew"] == "gemm2_wide_kernel"
+    # 16 rows: 128 experts x 16 tiles fill 256 CUs eight times, DS-V3's 32 x 28 only 3.5
+    assert names["qwen3_t512"] == "gemm2_wide_kernel" and names["ds_t1024"] == "gemm2_big_kernel"
+
+
 def test_gemm2_unit_figures_and_roofline_bound():
     # GEMM2: 2*I*H FLOPs per pair; W2 + S2 per active expert, bf16 C read and one bf16 row
     # written per pair

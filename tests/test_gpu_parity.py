@@ -384,6 +384,25 @@ def test_segment_length_boundaries(gpu, geom, T):
     assert ws["counts"].cpu().tolist() == counts
 
 
+@pytest.mark.parametrize("geom,T", [
+    # 128 x 256 tiles, the last one half outside H = 384; 64 and 256 expected rows
+    (Geometry(384, 384, 64, 64, 8, 1, 1, ROUTING_SOFTMAX, "wide-h384"), 512),
+    (Geometry(384, 384, 64, 64, 8, 1, 1, ROUTING_SOFTMAX, "wide-h384"), 2048),
+    # five or more rounds of tiles: 64 x 256 tiles in three slots (8 and 43 expected rows; as many K
+    # blocks as slots, and one more), 128 x 256 ones from 44
+    (Geometry(1152, 384, 256, 256, 8, 1, 1, ROUTING_SOFTMAX, "wide-e256"), 256),
+    (Geometry(1152, 384, 256, 256, 8, 1, 1, ROUTING_SOFTMAX, "wide-e256"), 1407),
+    (Geometry(1152, 384, 256, 256, 8, 1, 1, ROUTING_SOFTMAX, "wide-e256"), 1408),
+    (Geometry(1152, 512, 256, 256, 8, 1, 1, ROUTING_SOFTMAX, "wide-i512"), 320),
+], ids=lambda v: getattr(v, "name", v))
+def test_wide_gemm2_segment_boundaries(gpu, geom, T):
+    """The 256-column GEMM2 at segment lengths around every tile edge and empty experts."""
+    counts = boundary_counts(T, geom.num_experts)
+    lg = logits_for_counts(counts, T, geom.num_experts)
+    _, ws = check_case(geom, T, gpu, seed=9, logits=lg, bias=False, rsf=1.0)
+    assert ws["counts"].cpu().tolist() == counts
+
+
 SEG_WIDE = Geometry(256, 256, 256, 256, 8, 1, 1, ROUTING_SOFTMAX, "segments-wide")
 
 
