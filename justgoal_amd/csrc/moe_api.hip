@@ -257,9 +257,10 @@ int moe_run_ex(const moe_geometry* geom, const void* logits, const void* bias, c
   const int H = geom->hidden, I = geom->intermediate, El = geom->local_experts;
   const int Np = (int)max_pairs(geom, T);
   const int rows_hint = (int)((int64_t)T * geom->top_k / geom->num_experts);
+  const int pairs_hint = (int)((int64_t)T * geom->top_k * El / geom->num_experts);
   JG_TRY(jgmoe::launch_gemm1((const uint8_t*)hs, (const float*)hs_scale, (const uint8_t*)w13,
                              (const float*)s13, r.counts, r.offsets, r.sorted_tok, r.C, T, H, I,
-                             El, Np, rows_hint, stream));
+                             El, Np, rows_hint, pairs_hint, stream));
   JG_TRY(mark_stage(3, stream));
   JG_TRY(jgmoe::launch_gemm2(r.C, (const uint8_t*)w2, (const float*)s2, r.counts, r.offsets,
                              r.sorted_w, jgmoe::Gemm2Out{r.pair_dst, (uint16_t*)out, r.partial},

@@ -102,11 +102,11 @@ static inline int stream_mt(int rows_hint) { return rows_hint <= 16 ? 1 : rows_h
 hipError_t launch_gemm1(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,
                         const float* s13, const int32_t* counts, const int32_t* offsets,
                         const int32_t* sorted_tok, uint16_t* C, int T, int H, int I, int E_l,
-                        int max_pairs, int rows_hint, hipStream_t stream) {
+                        int max_pairs, int rows_hint, int pairs_hint, hipStream_t stream) {
   if (max_pairs <= 0) return hipSuccess;
   if (rows_hint <= kStreamMaxRows)
     return launch_gemm1_stream(hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I,
-                               E_l, max_pairs, stream_mt(rows_hint), stream);
+                               E_l, max_pairs, pairs_hint, stream_mt(rows_hint), stream);
   if (rows_hint >= kBigRows) {
     const hipError_t b = launch_gemm1_big(hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C,
                                           T, H, I, E_l, max_pairs, rows_hint, stream);
@@ -116,7 +116,7 @@ hipError_t launch_gemm1(const uint8_t* hs, const float* hs_scale, const uint8_t*
                                          T, H, I, E_l, max_pairs, stream);
   if (e != hipErrorNotSupported) return e;
   return launch_gemm1_stream(hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I, E_l,
-                             max_pairs, 4, stream);
+                             max_pairs, pairs_hint, 4, stream);
 }
 
 hipError_t launch_gemm2(const uint16_t* C, const uint8_t* w2, const float* s2,

@@ -28,11 +28,12 @@ int route_chunks(int T);
 
 // Grouped GEMM1 (W13) with the SwiGLU epilogue: C[p, :] = bf16(X1 * silu(X2)) for every pair p.
 // max_pairs bounds the number of pairs (sizes the grid; surplus workgroups exit at once);
-// rows_hint, the expected pairs per expert under uniform routing, picks the tile shape.
+// rows_hint and pairs_hint, the expected pairs per expert and over the local experts under uniform
+// routing, pick the tile shape.
 hipError_t launch_gemm1(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,
                         const float* s13, const int32_t* counts, const int32_t* offsets,
                         const int32_t* sorted_tok, uint16_t* C, int T, int H, int I, int E_l,
-                        int max_pairs, int rows_hint, hipStream_t stream);
+                        int max_pairs, int rows_hint, int pairs_hint, hipStream_t stream);
 
 // Grouped GEMM2 (W2): row = bf16(w_p * (C[p, :] @ W2[e]^T)), stored at the pair's destination
 // d = pair_dst[p]: out row d when d >= 0 (the token's first local pair in ascending expert
@@ -51,7 +52,8 @@ hipError_t launch_gemm2(const uint16_t* C, const uint8_t* w2, const float* s2,
 hipError_t launch_gemm1_stream(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,
                                const float* s13, const int32_t* counts, const int32_t* offsets,
                                const int32_t* sorted_tok, uint16_t* C, int T, int H, int I,
-                               int E_l, int max_pairs, int mt, hipStream_t stream);
+                               int E_l, int max_pairs, int pairs_hint, int mt,
+                               hipStream_t stream);
 hipError_t launch_gemm2_stream(const uint16_t* C, const uint8_t* w2, const float* s2,
                                const int32_t* counts, const int32_t* offsets,
                                const float* sorted_w, Gemm2Out dst, int H, int I, int E_l,

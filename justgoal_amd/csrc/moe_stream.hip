@@ -6,7 +6,8 @@
 //
 // * Work items are per wave: (M-tile of 16*MT pairs, 16 output columns, full K). Each wave loops
 //   over its items (persistent grid, items dealt wave-index major); there is no workgroup
-//   synchronisation.
+//   synchronisation. GEMM1's items may instead belong to a workgroup, each of its four waves taking
+//   a quarter of K, with a reduction through LDS at the end of an item.
 // * Weight K-blocks (16 rows x 128 bytes per matrix) go global -> LDS by DMA into a per-wave ring
 //   of D slots, two instructions per block, each fetching 8 rows as whole 128-byte lines
 //   (register-staged MFMA operands would touch every line twice). The activation rows of the
@@ -70,7 +71,7 @@ struct G1Item {
   int m0, cnt, seg, c0;
 };
 
-template <int MT, int D>
+template <int MT, int D, int KS>
 __global__ __launch_bounds__(256) void gemm1_stream_kernel(
     const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale,
     const uint8_t* __restrict__ w13, const float* __restrict__ s13,
@@ -79,17 +80,21 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
     int E_l) {
   constexpr int BM = 16 * MT;
   constexpr int OPS = 3 * MT + 4;  // vector-memory operations per K step
+  static_assert(KS == 1 || KS == kWavesPerGroup, "K is split over the workgroup's waves or not");
   __shared__ __attribute__((aligned(16))) uint8_t ring[kWavesPerGroup][D][2 * kWBlk];
+  // KS > 1: partial sums of an item, double buffered by item parity
+  __shared__ __attribute__((aligned(16))) v4f red[KS > 1 ? 2 : 1][KS > 1 ? KS : 1][2 * MT][kWave];
 
   const int lane = threadIdx.x & (kWave - 1), w = wave_id();
   const int r16 = lane & 15, g = lane >> 4;
   const int NCT = I / 16, NKB = H / kBlock;
+  const int nkb = NKB / KS, kfirst = KS > 1 ? w * nkb : 0;  // this wave's K blocks
   TileMap tm;
   tm.init(counts, offsets, E_l, BM);
   const int items = tm.total * NCT;
-  const int stride = gridDim.x * kWavesPerGroup;
-  int it = __builtin_amdgcn_readfirstlane(first_item(w));
-  if (it >= items) return;
+  const int stride = KS > 1 ? gridDim.x : gridDim.x * kWavesPerGroup;
+  int it = __builtin_amdgcn_readfirstlane(KS > 1 ? (int)blockIdx.x : first_item(w));
+  if (it >= items) return;  // KS > 1: the whole workgroup
 
   const __amdgpu_buffer_rsrc_t ares = make_rsrc(hs, (uint32_t)T * H);
   const __amdgpu_buffer_rsrc_t sares = make_rsrc(hs_scale, (uint32_t)T * NKB * 4);
@@ -134,11 +139,12 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
   finish(nxt, tok);
 
   G1Slot<MT> sl[D];
-  // Issue K block kbi of item cur (or nxt when `second`) into slot d. After a wave's last item
-  // there is no next item: those prefetches keep the step's operation count (the counted waits
+  // Issue this wave's K block kbl of item cur (or nxt when `second`) into slot d. After a wave's
+  // last item there is no next item: those prefetches keep the step's operation count (the counted waits
   // rely on it) but use an out-of-range offset, so they return zeros and fetch nothing.
-  auto issue = [&](bool second, int kbi, G1Slot<MT>& s, int d) {
+  auto issue = [&](bool second, int kbl, G1Slot<MT>& s, int d) {
     const bool dead = uniform(second && it_n >= items);
+    const int kbi = kfirst + kbl;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const uint32_t ao = dead ? kNoFetch : second ? nxt.aoff[mt] : cur.aoff[mt];
@@ -169,6 +175,7 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
   retire(nxt.sc2.v0);
   retire(nxt.sc2.v1);
 
+  int turn = 0;
   for (;;) {
     // Token ids and scales of the item after nxt, consumed one item from now.
     const int it_nn = it_n + stride;
@@ -183,7 +190,7 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
     // do-while: the compiler must see that the trip (with its retires) runs at least once
     int kb0 = 0;
     do {
-      const bool last = kb0 + D >= NKB;  // this trip's prefetches belong to the next item
+      const bool last = kb0 + D >= nkb;  // this trip's prefetches belong to the next item
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         const int kb = kb0 + d;
@@ -196,7 +203,7 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
                            (int)x1h[0], (int)x1h[1], (int)x1h[2], (int)x1h[3]};
         const v8i b2 = v8i{(int)x2l[0], (int)x2l[1], (int)x2l[2], (int)x2l[3],
                            (int)x2h[0], (int)x2h[1], (int)x2h[2], (int)x2h[3]};
-        const float sw1 = cur.sc1.get(kb), sw2 = cur.sc2.get(kb);
+        const float sw1 = cur.sc1.get(kfirst + kb), sw2 = cur.sc2.get(kfirst + kb);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           const float f1 = sl[d].sa[mt] * sw1, f2 = sl[d].sa[mt] * sw2;
@@ -209,7 +216,7 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
           }
         }
         __builtin_amdgcn_sched_barrier(0);
-        issue(last, last ? kb + D - NKB : kb + D, sl[d], d);
+        issue(last, last ? kb + D - nkb : kb + D, sl[d], d);
         __builtin_amdgcn_sched_barrier(0);
       }
       // The next-but-one item's metadata loads are long complete here; retiring them now
@@ -221,12 +228,45 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) retire(tok[mt]);
       kb0 += D;
-    } while (kb0 < NKB);
+    } while (kb0 < nkb);
 
+    // KS > 1: every wave leaves its partial sums in LDS, and after one barrier the waves in turn
+    // (wave n % KS for the workgroup's n-th item) add them up in wave order and store. The buffer of
+    // item n is written again for item n + 2, past the barrier of item n + 1.
+    bool store = true;
+    if constexpr (KS > 1) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        red[turn & 1][w][2 * mt][lane] = acc1[mt];
+        red[turn & 1][w][2 * mt + 1][lane] = acc2[mt];
+      }
+      lds_wait_all();
+      __builtin_amdgcn_s_barrier();  // (a bare one: a fence would wait for every DMA in flight)
+      store = w == turn % KS;
+      if (store) {
+        v4u part[KS][2 * MT];
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+          for (int j = 0; j < 2 * MT; ++j)
+            part[k][j] = ds_read16(lds_addr(&red[turn & 1][k][j][lane]));
+        lds_wait_all();
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+          for (int j = 0; j < 2 * MT; ++j) {
+            lds_fence(part[k][j]);
+            v4f& acc = (j & 1) ? acc2[j / 2] : acc1[j / 2];
+            const v4f v = __builtin_bit_cast(v4f, part[k][j]);
+            acc = k == 0 ? v : acc + v;
+          }
+      }
+      ++turn;
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int r = cur.m0 + mt * 16 + r16;
-      if (r < cur.cnt) {
+      if (store && r < cur.cnt) {
         uint32_t h[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -454,35 +494,58 @@ static inline int ring_depth(int nkb, int dmax) {
 constexpr int kG1StreamD = 8;
 constexpr int kG2StreamD = 8;
 
+// GEMM1 items split over the K quarters of a workgroup's four waves (KS = 4). A wave then fetches a
+// contiguous quarter of each weight row, the four side by side, instead of 1 KiB windows of 16
+// rows far from its neighbours': with the 4 KiB row pitch of H = 4096 the unsplit form keeps
+// hitting few memory channels (Qwen3-style GEMM1 stage T=8 114 -> 98 us, T=16 177 -> 154, T=32 237 ->
+// 208, T=64 270 -> 237: 6.8 TB/s, the rate of a plain non-temporal read). It also gives a
+// batch of few items four times as many, so that no CU is left with one wave's loads in flight
+// (DS-V3 T=1 call 33.3 -> 31.0 us), and evens out the last round (DS-V3 T=48 90.1 -> 88.1, T=128 126.4
+// -> 125.0). From half to one and a half whole-K items per wave that the chip holds the split only
+// adds its reduction (Qwen3-style T=1 43.9 against 44.6 us, T=2 62.1 against 64.2; DS-V3 T=7 46.6
+// against 47.0), so there K stays whole. `expected` counts items under uniform routing.
+
 hipError_t launch_gemm1_stream(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,
                                const float* s13, const int32_t* counts, const int32_t* offsets,
                                const int32_t* sorted_tok, uint16_t* C, int T, int H, int I,
-                               int E_l, int max_pairs, int mt, hipStream_t stream) {
+                               int E_l, int max_pairs, int pairs_hint, int mt,
+                               hipStream_t stream) {
   const int nkb = H / kBlock;
-#define JG_G1S(MT, D)                                                                          \
+  const long long expected = (long long)(pairs_hint < E_l ? pairs_hint : E_l) * (I / 16);
+  const long long waves = (long long)kWavesPerGroup * device_cu_count();
+  const bool split = 2 * expected < waves || 2 * expected > 3 * waves;
+#define JG_G1S(MT, D, KS)                                                                      \
   {                                                                                            \
-    const long long waves = max_m_tiles(max_pairs, 16 * MT, E_l) * (I / 16);                   \
+    const long long tiles = max_m_tiles(max_pairs, 16 * MT, E_l) * (I / 16);                   \
     const int grid = persistent_grid(groups_per_cu(kWavesPerGroup * D * 2 * kWBlk),            \
-                                     (waves + kWavesPerGroup - 1) / kWavesPerGroup);            \
-    gemm1_stream_kernel<MT, D><<<grid, kWavesPerGroup * kWave, 0, stream>>>(                   \
+                                     (tiles * KS + kWavesPerGroup - 1) / kWavesPerGroup);       \
+    gemm1_stream_kernel<MT, D, KS><<<grid, kWavesPerGroup * kWave, 0, stream>>>(               \
         hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I, E_l);                 \
     return hipGetLastError();                                                                  \
   }
   const int d = ring_depth(nkb, mt == 1 ? kG1StreamD : 4);
   if (mt == 1) {
-    if (d >= 8) JG_G1S(1, 8)
-    if (d == 4) JG_G1S(1, 4)
-    if (d == 2) JG_G1S(1, 2)
-    JG_G1S(1, 1)
+    if (split && nkb % kWavesPerGroup == 0) {
+      const int n = nkb / kWavesPerGroup;
+      if (n % 8 == 0) JG_G1S(1, 8, 4)
+      if (n % 7 == 0) JG_G1S(1, 7, 4)
+      if (n % 6 == 0) JG_G1S(1, 6, 4)
+      if (n % 5 == 0) JG_G1S(1, 5, 4)
+      if (n % 4 == 0) JG_G1S(1, 4, 4)
+    }
+    if (d >= 8) JG_G1S(1, 8, 1)
+    if (d == 4) JG_G1S(1, 4, 1)
+    if (d == 2) JG_G1S(1, 2, 1)
+    JG_G1S(1, 1, 1)
   }
   if (mt == 2) {
-    if (d == 4) JG_G1S(2, 4)
-    if (d == 2) JG_G1S(2, 2)
-    JG_G1S(2, 1)
+    if (d == 4) JG_G1S(2, 4, 1)
+    if (d == 2) JG_G1S(2, 2, 1)
+    JG_G1S(2, 1, 1)
   }
-  if (d == 4) JG_G1S(4, 4)
-  if (d == 2) JG_G1S(4, 2)
-  JG_G1S(4, 1)
+  if (d == 4) JG_G1S(4, 4, 1)
+  if (d == 2) JG_G1S(4, 2, 1)
+  JG_G1S(4, 1, 1)
 #undef JG_G1S
 }
 

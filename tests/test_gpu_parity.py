@@ -403,6 +403,21 @@ def test_wide_gemm2_segment_boundaries(gpu, geom, T):
     assert ws["counts"].cpu().tolist() == counts
 
 
+@pytest.mark.parametrize("T", [1, 32])
+@pytest.mark.parametrize("H", [2048, 2560, 3072, 3584, 4096])
+def test_streaming_gemm1_split_over_k(gpu, H, T):
+    """The streaming GEMM1 with K split over a workgroup's waves, at each of its ring depths
+    (4..8 blocks per wave): one token, and segments of 0, 1, 2, 15-17, 31 and 32 pairs."""
+    geom = Geometry(H, 512, 64, 64, 8, 1, 1, ROUTING_SOFTMAX, f"split-h{H}")
+    lg = None
+    if T > 1:
+        counts = boundary_counts(T)
+        lg = logits_for_counts(counts, T, geom.num_experts)
+    _, ws = check_case(geom, T, gpu, seed=9, logits=lg, bias=False, rsf=1.0)
+    if T > 1:
+        assert ws["counts"].cpu().tolist() == counts
+
+
 SEG_WIDE = Geometry(256, 256, 256, 256, 8, 1, 1, ROUTING_SOFTMAX, "segments-wide")
 
 
