@@ -50,12 +50,13 @@ struct B1Scalars {
   const uint8_t* wbase;  // the expert's W13
   uint32_t c0;           // first C column of the tile
   int e, m0, cnt, seg;
+  int rot;               // K rotation (ROT)
 };
 
 // MS: 16-row sub-tiles per compute wave (BM = 32*MS); NS: 16-column sub-tiles (BN = 32*NS).
 // MS/NS: 16-row/16-column sub-tiles per compute wave; WM x WN compute waves (wave index w:
 // wm = w % WM, wn = w / WM), so BM = 16*MS*WM and BN = 16*NS*WN; wave WM*WN is the producer.
-template <int MS, int NS, int D, int WM, int WN>
+template <int MS, int NS, int D, int WM, int WN, bool ROT>
 __global__ __launch_bounds__((WM * WN + 1) * kWave) void gemm1_big_kernel(
     const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale,
     const uint8_t* __restrict__ w13, const float* __restrict__ s13,
@@ -93,6 +94,7 @@ __global__ __launch_bounds__((WM * WN + 1) * kWave) void gemm1_big_kernel(
     x.cnt = uniform(x.cnt);
     x.seg = uniform(x.seg);
     x.c0 = uniform((uint32_t)(nt * BN));
+    x.rot = ROT ? uniform(k_rotation(nt, NKB)) : 0;
     x.wbase = uniform(w13 + (size_t)x.e * 2 * I * H);
   };
   int it_n = it + stride;
@@ -149,6 +151,7 @@ __global__ __launch_bounds__((WM * WN + 1) * kWave) void gemm1_big_kernel(
     finish(nxt);
 
     auto issue = [&](const P& x, int kbi, int slot) {
+      if constexpr (ROT) kbi = rotated(kbi, uniform(x.s.rot), NKB);
 #pragma unroll
       for (int j = 0; j < AI; ++j)
         dma16(ares, &aring[slot][j * 1024], x.aoff[j],
@@ -318,7 +321,8 @@ __global__ __launch_bounds__((WM * WN + 1) * kWave) void gemm1_big_kernel(
     do {
       const int d = slot, dn = slot + 1 == D ? 0 : slot + 1;
       const uint32_t ab = a_base(d), bb = b_base(d);
-      const float sw1 = cur.sc1.get(kb), sw2 = cur.sc2.get(kb);
+      const int kr = ROT ? rotated(kb, uniform(cur.s.rot), NKB) : kb;
+      const float sw1 = cur.sc1.get(kr), sw2 = cur.sc2.get(kr);
       lds_wait_all();  // the head fragments (read during the previous step) have landed
       fence_a(0);
       fence_a(1);
@@ -796,6 +800,10 @@ constexpr int kB1ShortMs = 2;
 // 240.9, T=6144 248.7 against 256.6, T=8192 334.5 against 341.3, T=16384 skewed 1922 against
 // 2006. The same 2 x 2 layout measured within 1% for the 64-row tiles of both GEMMs.
 constexpr int kB1EightWaveRows = 160;
+// The K rotation of k_rotation (moe_device.h) below 112 expected rows: with a second M-tile per
+// expert it parts the workgroups that share a weight panel in L2 (Qwen3-style call T=1024 524.1 ->
+// 507.0 us, T=1536 585.5 -> 558.5, but T=2048, 128 rows, 749.9 -> 763.8).
+constexpr int kB1RotateRows = 112;
 constexpr int kB1WideNs = 4;
 constexpr int kB1WideWm = 2;
 constexpr int kB1WideWn = 2;
@@ -808,7 +816,7 @@ constexpr int kB2Wm = 2;
 constexpr int kB2Wn = 4;
 constexpr int kB2D = 4;
 
-template <int MS, int NS, int D, int WM, int WN>
+template <int MS, int NS, int D, int WM, int WN, bool ROT>
 static hipError_t launch_gemm1_big_t(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,
                                      const float* s13, const int32_t* counts,
                                      const int32_t* offsets, const int32_t* sorted_tok,
@@ -818,7 +826,7 @@ static hipError_t launch_gemm1_big_t(const uint8_t* hs, const float* hs_scale, c
   if (I % BN != 0 || H / kBlock < D - 1 || (int64_t)T * H >= kOutOfRange)
     return hipErrorNotSupported;
   const int grid = big_grid(big_tiles(max_pairs, 16 * MS * WM, E_l) * (I / BN));
-  gemm1_big_kernel<MS, NS, D, WM, WN><<<grid, (WM * WN + 1) * kWave, 0, stream>>>(
+  gemm1_big_kernel<MS, NS, D, WM, WN, ROT><<<grid, (WM * WN + 1) * kWave, 0, stream>>>(
       hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I, E_l, max_pairs,
       gemm1_sched(I / BN));
   return hipGetLastError();
@@ -828,15 +836,18 @@ hipError_t launch_gemm1_big(const uint8_t* hs, const float* hs_scale, const uint
                             const float* s13, const int32_t* counts, const int32_t* offsets,
                             const int32_t* sorted_tok, uint16_t* C, int T, int H, int I, int E_l,
                             int max_pairs, int rows_hint, hipStream_t stream) {
+  const bool rotate = rows_hint < kB1RotateRows && H / kBlock % kRotPitchBlocks == 0;
+#define JG_G1B(MS, NS, WM, WN, ROT)                                                              \
+  launch_gemm1_big_t<MS, NS, kB1D, WM, WN, ROT>(hs, hs_scale, w13, s13, counts, offsets,         \
+                                                sorted_tok, C, T, H, I, E_l, max_pairs, stream)
   if (rows_hint < kB1TallRows)
-    return launch_gemm1_big_t<kB1ShortMs, kB1Ns, kB1D, kB1Wm, kB1Wn>(
-        hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I, E_l, max_pairs, stream);
+    return rotate ? JG_G1B(kB1ShortMs, kB1Ns, kB1Wm, kB1Wn, true)
+                  : JG_G1B(kB1ShortMs, kB1Ns, kB1Wm, kB1Wn, false);
   if (rows_hint < kB1EightWaveRows)
-    return launch_gemm1_big_t<kB1Ms, kB1WideNs, kB1D, kB1WideWm, kB1WideWn>(
-        hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I, E_l, max_pairs, stream);
-  return launch_gemm1_big_t<kB1Ms, kB1Ns, kB1D, kB1Wm, kB1Wn>(hs, hs_scale, w13, s13, counts,
-                                                              offsets, sorted_tok, C, T, H, I,
-                                                              E_l, max_pairs, stream);
+    return rotate ? JG_G1B(kB1Ms, kB1WideNs, kB1WideWm, kB1WideWn, true)
+                  : JG_G1B(kB1Ms, kB1WideNs, kB1WideWm, kB1WideWn, false);
+  return JG_G1B(kB1Ms, kB1Ns, kB1Wm, kB1Wn, false);
+#undef JG_G1B
 }
 
 template <int MS, int NS, int D, int WM, int WN>

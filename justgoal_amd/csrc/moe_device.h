@@ -425,6 +425,22 @@ __device__ __forceinline__ int map_item(const TileMapLds& tml, int item, int ite
   return e;
 }
 
+// Rotation of a tile's K order. Workgroups step through K side by side, so at any time they fetch
+// about the same K columns of many weight rows. With a row pitch that is a multiple of 4 KiB those
+// addresses fall on few memory channels; tile nt of the N-tiles then starts 5 nt blocks
+// later (5 is coprime to every block count this applies to) and wraps around, which spreads them.
+// GEMM1 stage, H = 4096 (Qwen3-style): T=128 282 -> 252 us, T=512 290 -> 266, T=1024 312 -> 289, T=1536
+// 333 -> 297; H = 8192 T=512 526 -> 495. Other pitches gain nothing (2048, 3072, 5120 and 6144:
+// within 1%) or lose where M-tiles share activation rows in L2 (DS-V3's 7168, T=14107: 307 -> 342),
+// so they keep the plain order.
+constexpr int kRotPitchBlocks = 4096 / kBlock;
+__device__ __forceinline__ int k_rotation(int nt, int nkb) { return (5 * nt) % nkb; }
+// The K block that a tile with rotation rot takes as its kb-th.
+__device__ __forceinline__ int rotated(int kb, int rot, int nkb) {
+  const int k = kb + rot;
+  return k >= nkb ? k - nkb : k;
+}
+
 // Total M-tiles over all experts: sum of ceil(count / bm). Wave-uniform; every lane must call.
 __device__ __forceinline__ int count_m_tiles(const int32_t* __restrict__ counts, int n_experts,
                                              int bm) {

@@ -42,9 +42,10 @@ struct T1Item {
   uint32_t aoff[MT / 2];  // per lane: global offset of its A DMA chunk (token row, K 0)
   uint32_t saoff;         // per lane: token * 4 for its activation-scale DMA
   int m0, cnt, seg, c0;
+  int rot;                // K rotation (ROT)
 };
 
-template <int MT, int D>
+template <int MT, int D, bool ROT>
 __global__ __launch_bounds__(256) void gemm1_tile_kernel(
     const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale,
     const uint8_t* __restrict__ w13, const float* __restrict__ s13,
@@ -97,6 +98,7 @@ __global__ __launch_bounds__(256) void gemm1_tile_kernel(
     x.cnt = uniform(x.cnt);
     x.seg = uniform(x.seg);
     x.c0 = uniform(nt * 64 + w * 16);
+    x.rot = ROT ? uniform(k_rotation(nt, NKB)) : 0;
     x.wbase = uniform(w13 + (size_t)e * 2 * I * H);
     x.wsoff = uniform((uint32_t)x.c0 * H);
     const int last = x.cnt - 1;
@@ -148,6 +150,7 @@ __global__ __launch_bounds__(256) void gemm1_tile_kernel(
   finish(nxt);
 
   auto issue = [&](bool second, int kbi, int slot) {
+    if constexpr (ROT) kbi = rotated(kbi, uniform(second ? nxt.rot : cur.rot), NKB);
 #pragma unroll
     for (int i = 0; i < AI; ++i)
       dma16(ares, &aring[slot][(w * AI + i) * 1024], second ? nxt.aoff[i] : cur.aoff[i],
@@ -217,7 +220,8 @@ __global__ __launch_bounds__(256) void gemm1_tile_kernel(
                            (int)x1h[0], (int)x1h[1], (int)x1h[2], (int)x1h[3]};
         const v8i b2 = v8i{(int)x2l[0], (int)x2l[1], (int)x2l[2], (int)x2l[3],
                            (int)x2h[0], (int)x2h[1], (int)x2h[2], (int)x2h[3]};
-        const float sw1 = cur.sc1.get(kb), sw2 = cur.sc2.get(kb);
+        const int kr = ROT ? rotated(kb, uniform(cur.rot), NKB) : kb;
+        const float sw1 = cur.sc1.get(kr), sw2 = cur.sc2.get(kr);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           lds_fence(al[mt]);
@@ -523,7 +527,9 @@ hipError_t launch_gemm1_tile(const uint8_t* hs, const float* hs_scale, const uin
                         D * (MT < 4 ? kWave : 16 * MT) * 4 + kWaves * (MT / 2 + 5) * kWave * 4;  \
     const int grid =                                                                            \
         tile_grid(tile_groups_per_cu(lds), tile_count(max_pairs, 16 * MT, E_l) * (I / 64));     \
-    gemm1_tile_kernel<MT, D><<<grid, kWaves * kWave, 0, stream>>>(                              \
+    const auto kernel = H / kBlock % kRotPitchBlocks == 0 ? gemm1_tile_kernel<MT, D, true>      \
+                                                          : gemm1_tile_kernel<MT, D, false>;    \
+    kernel<<<grid, kWaves * kWave, 0, stream>>>(                                                \
         hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I, E_l, max_pairs);       \
     return hipGetLastError();                                                                   \
   }

@@ -418,6 +418,16 @@ def test_streaming_gemm1_split_over_k(gpu, H, T):
         assert ws["counts"].cpu().tolist() == counts
 
 
+# H = 4096: a row pitch of 4 KiB, where GEMM1's tiles rotate their K order (LDS-tiled at 6 expected
+# rows; 64-row and 128-row large tiles at 16 and 96; 128 rows no longer rotate)
+@pytest.mark.parametrize("T", [48, 128, 768, 1024])
+def test_rotated_k_order(gpu, T):
+    geom = Geometry(4096, 256, 64, 64, 8, 1, 1, ROUTING_SOFTMAX, "rotated-h4096")
+    counts = boundary_counts(T)
+    lg = logits_for_counts(counts, T, geom.num_experts)
+    check_case(geom, T, gpu, seed=9, logits=lg, bias=False, rsf=1.0)
+
+
 SEG_WIDE = Geometry(256, 256, 256, 256, 8, 1, 1, ROUTING_SOFTMAX, "segments-wide")
 
 
