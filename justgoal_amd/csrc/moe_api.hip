@@ -141,6 +141,16 @@ int route_and_permute(const moe_geometry* g, const void* logits, const void* bia
                       int local_offset, float scaling, const Regions& r, int T,
                       hipStream_t stream) {
   JG_TRY(mark_stage(0, stream));
+  const hipError_t fused = jgmoe::launch_route_permute(
+      (const float*)logits, (const uint16_t*)bias, T, g->num_experts, g->n_group, g->topk_group,
+      g->top_k, g->routing_method, scaling, local_offset, g->local_experts, r.topk_idx, r.topk_w,
+      r.hist, r.counts, r.offsets, r.sorted_tok, r.sorted_w, r.pair_dst, r.pair_of, stream);
+  if (fused != hipErrorNotSupported) {
+    JG_TRY(fused);
+    JG_TRY(mark_stage(1, stream));
+    JG_TRY(mark_stage(2, stream));
+    return MOE_OK;
+  }
   JG_TRY(jgmoe::launch_route((const float*)logits, (const uint16_t*)bias, T, g->num_experts,
                              g->n_group, g->topk_group, g->top_k, g->routing_method, scaling,
                              local_offset, g->local_experts, r.topk_idx, r.topk_w, r.hist,

@@ -22,6 +22,14 @@ hipError_t launch_permute(const int32_t* topk_idx, const float* topk_w, const in
                           int32_t* offsets, int32_t* sorted_tok, float* sorted_w,
                           int32_t* pair_dst, int32_t* pair_of, hipStream_t stream);
 
+// Both in one launch, for batches of a few tokens; hipErrorNotSupported above.
+hipError_t launch_route_permute(const float* logits, const uint16_t* bias, int T, int E, int n_group,
+                                int topk_group, int top_k, int method, float rsf, int local_offset,
+                                int E_l, int32_t* topk_idx, float* topk_w, int32_t* hist,
+                                int32_t* counts, int32_t* offsets, int32_t* sorted_tok,
+                                float* sorted_w, int32_t* pair_dst, int32_t* pair_of,
+                                hipStream_t stream);
+
 // Number of routing workgroups (4 tokens each up to T = 2048, 16 above) = rows of the chunk count
 // table.
 int route_chunks(int T);

@@ -12,6 +12,8 @@
 //   followed by a ballot that picks the lowest lane (= lowest expert index) holding it.
 //   Each workgroup also writes its per-expert pair counts (one row of the chunk count table).
 //
+// route_permute_kernel: both in one launch, for batches of up to 12 (softmax: 16) tokens.
+//
 // permute_kernel: one workgroup per 64 tokens. From the count rows it derives the segment
 //   offsets and this chunk's base inside each segment, then places its pairs: a pair's rank
 //   inside its expert is a popcount over a per-expert token bitmask built with LDS atomic ORs
@@ -34,6 +36,10 @@ constexpr int kRouteWaves = 16;          // most tokens per routing workgroup (o
 constexpr int kRouteSmallT = 2048, kRouteWavesSmall = 4;
 __host__ __device__ __forceinline__ int route_tokens_per_group(int T) {
   return T <= kRouteSmallT ? kRouteWavesSmall : kRouteWaves;
+}
+__host__ __device__ __forceinline__ int route_chunks_of(int T) {
+  const int tpw = route_tokens_per_group(T);
+  return (T + tpw - 1) / tpw;
 }
 constexpr int kPlaceTokens = 64;         // tokens per permute workgroup (one bitmask word)
 constexpr int kMaxLocal = 256;           // local experts supported by the count / scan stages
@@ -334,22 +340,16 @@ __device__ __forceinline__ void wave_exclusive_scan(const int* in, int* out, int
   if (lane == kWave - 1) out[n] = incl;
 }
 
-}  // namespace
-
+// One wave routes token t (if t < T) and leaves its pairs in row `row` of tp.
 template <int VPL, int METHOD>
-__global__ __launch_bounds__(1024) void route_kernel(
-    const float* __restrict__ logits, const uint16_t* __restrict__ bias, int T, int n_group,
-    int topk_group, int top_k, float rsf, int local_offset, int E_l, int32_t* __restrict__ topk_idx,
-    float* __restrict__ topk_w, int32_t* __restrict__ hist) {
+__device__ __forceinline__ void route_into(const float* __restrict__ logits,
+                                           const uint16_t* __restrict__ bias, int t, int T, int row,
+                                           int n_group, int topk_group, int top_k, float rsf,
+                                           int local_offset, int E_l,
+                                           int32_t* __restrict__ topk_idx,
+                                           float* __restrict__ topk_w, TokenPairs& tp) {
   constexpr int E = VPL * kWave;
-  __shared__ TokenPairs tp;  // rows 0..tpw-1 used
-  __shared__ ExpertMasks masks;
-  __shared__ int cnt[kMaxLocal];
-  const int lane = threadIdx.x & (kWave - 1), wave = wave_id();
-  const int tpw = blockDim.x / kWave;  // tokens of this workgroup
-  const int t0 = blockIdx.x * tpw;
-  const int t = t0 + wave;
-
+  const int lane = threadIdx.x & (kWave - 1);
   int le = -1;
   float w = 0.f;
   if (t < T) {  // wave-uniform
@@ -368,12 +368,63 @@ __global__ __launch_bounds__(1024) void route_kernel(
     }
   }
   if (lane < kMaxTopK) {
-    tp.le[wave][lane] = le;
-    tp.w[wave][lane] = w;
+    tp.le[row][lane] = le;
+    tp.w[row][lane] = w;
   }
+}
+
+}  // namespace
+
+template <int VPL, int METHOD>
+__global__ __launch_bounds__(1024) void route_kernel(
+    const float* __restrict__ logits, const uint16_t* __restrict__ bias, int T, int n_group,
+    int topk_group, int top_k, float rsf, int local_offset, int E_l, int32_t* __restrict__ topk_idx,
+    float* __restrict__ topk_w, int32_t* __restrict__ hist) {
+  __shared__ TokenPairs tp;  // rows 0..tpw-1 used
+  __shared__ ExpertMasks masks;
+  __shared__ int cnt[kMaxLocal];
+  const int wave = wave_id();
+  const int tpw = blockDim.x / kWave;  // tokens of this workgroup
+  route_into<VPL, METHOD>(logits, bias, blockIdx.x * tpw + wave, T, wave, n_group, topk_group, top_k,
+                          rsf, local_offset, E_l, topk_idx, topk_w, tp);
   __syncthreads();
   build_masks(tp, tpw, top_k, E_l, masks, cnt);
   for (int e = threadIdx.x; e < E_l; e += blockDim.x) hist[(size_t)blockIdx.x * E_l + e] = cnt[e];
+}
+
+// Routing and permute of a batch that fits one workgroup (one wave per token), in one launch: the
+// counts, segment offsets and placement come straight from the workgroup's own picks. Writes
+// everything route_kernel and permute_kernel write.
+template <int VPL, int METHOD>
+__global__ __launch_bounds__(1024) void route_permute_kernel(
+    const float* __restrict__ logits, const uint16_t* __restrict__ bias, int T, int n_group,
+    int topk_group, int top_k, float rsf, int local_offset, int E_l, int32_t* __restrict__ topk_idx,
+    float* __restrict__ topk_w, int32_t* __restrict__ hist, int32_t* __restrict__ counts,
+    int32_t* __restrict__ offsets, int32_t* __restrict__ sorted_tok, float* __restrict__ sorted_w,
+    int32_t* __restrict__ pair_dst, int32_t* __restrict__ pair_of) {
+  __shared__ TokenPairs tp;
+  __shared__ ExpertMasks masks;
+  __shared__ int cnt[kMaxLocal];
+  __shared__ int off[kMaxLocal + 1];
+  const int wave = wave_id();
+  route_into<VPL, METHOD>(logits, bias, wave, T, wave, n_group, topk_group, top_k, rsf, local_offset,
+                          E_l, topk_idx, topk_w, tp);
+  __syncthreads();
+  build_masks(tp, T, top_k, E_l, masks, cnt);
+  if (wave == 0) wave_exclusive_scan(cnt, off, E_l);
+  __syncthreads();
+  for (int i = threadIdx.x; i <= E_l; i += blockDim.x) {
+    offsets[i] = off[i];
+    if (i < E_l) counts[i] = cnt[i];
+  }
+  // the chunk count rows (4 tokens each), as route_kernel leaves them
+  for (int i = threadIdx.x; i < route_chunks_of(T) * E_l; i += blockDim.x) {
+    const int r0 = i / E_l * kRouteWavesSmall;
+    const unsigned long long four = masks.bits[i % E_l][0] >> r0 & ((1ull << kRouteWavesSmall) - 1);
+    hist[i] = __popcll(four);
+  }
+  place_from_masks(tp, masks, T, 0, T, top_k, off, min(top_k, E_l), sorted_tok, sorted_w, pair_dst,
+                   pair_of);
 }
 
 __global__ __launch_bounds__(256) void permute_kernel(
@@ -478,9 +529,38 @@ __global__ __launch_bounds__(256) void permute_kernel(
                    pair_of);
 }
 
-int route_chunks(int T) {
-  const int tpw = route_tokens_per_group(T);
-  return (T + tpw - 1) / tpw;
+int route_chunks(int T) { return route_chunks_of(T); }
+
+// One launch for batches that one workgroup routes with a wave per token: up to 16 tokens, with
+// sigmoid routing, four of whose waves fill a SIMD's issue slots, up to 12. Whole call against the
+// two launches: DS-V3 T=1 31.1 -> 29.2 us, T=4 34.9 -> 32.8, T=7 46.7 -> 45.2, T=10 71.1 -> 70.2 (T=16
+// 70.7 -> 71.1); Qwen3-style T=1 44.2 -> 42.0, T=8 160.1 -> 158.0, T=16 240.1 -> 238.6.
+constexpr int kFusedRouteTSoftmax = kRouteWaves, kFusedRouteTSigmoid = 12;
+
+hipError_t launch_route_permute(const float* logits, const uint16_t* bias, int T, int E, int n_group,
+                                int topk_group, int top_k, int method, float rsf, int local_offset,
+                                int E_l, int32_t* topk_idx, float* topk_w, int32_t* hist,
+                                int32_t* counts, int32_t* offsets, int32_t* sorted_tok,
+                                float* sorted_w, int32_t* pair_dst, int32_t* pair_of,
+                                hipStream_t stream) {
+  if (E_l > kMaxLocal || top_k > kMaxTopK) return hipErrorInvalidValue;
+  if (T > (method == ROUTING_DS ? kFusedRouteTSigmoid : kFusedRouteTSoftmax))
+    return hipErrorNotSupported;
+#define JG_ROUTE(VPL)                                                                            \
+  if (E == VPL * kWave) {                                                                        \
+    const auto kernel = method == ROUTING_DS ? route_permute_kernel<VPL, ROUTING_DS>             \
+                                             : route_permute_kernel<VPL, ROUTING_SOFTMAX>;       \
+    kernel<<<1, T * kWave, 0, stream>>>(logits, bias, T, n_group, topk_group, top_k, rsf,        \
+                                        local_offset, E_l, topk_idx, topk_w, hist, counts,       \
+                                        offsets, sorted_tok, sorted_w, pair_dst, pair_of);       \
+    return hipGetLastError();                                                                    \
+  }
+  JG_ROUTE(1)
+  JG_ROUTE(2)
+  JG_ROUTE(4)
+  JG_ROUTE(8)
+#undef JG_ROUTE
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_route(const float* logits, const uint16_t* bias, int T, int E, int n_group,

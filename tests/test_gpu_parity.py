@@ -585,6 +585,19 @@ def test_route_entry_matches_oracle(gpu, geom, T, off):
                                   p["sorted_w"].view(np.uint32))
 
 
+EXPERTS_512 = Geometry(256, 256, 512, 64, 8, 8, 4, ROUTING_DS, "experts-512")
+
+
+@pytest.mark.parametrize("geom,T,off", [(DS_V3, 2, 32), (DS_V3, 11, 0), (DS_V3, 12, 64),
+                                        (DS_V3, 13, 64), (SMALL_GROUPS, 12, 16),
+                                        (EXPERTS_512, 9, 448), (QWEN3, 3, 0), (QWEN3, 15, 0),
+                                        (QWEN3, 16, 0), (QWEN3, 17, 0)],
+                         ids=lambda v: getattr(v, "name", v))
+def test_route_in_one_launch_matches_oracle(gpu, geom, T, off):
+    """Both sides of the batch sizes that route and permute in one launch."""
+    test_route_entry_matches_oracle(gpu, geom, T, off)
+
+
 # The operator captured in a HIP graph (serving loops replay one): the library records no memset
 # or allocation, so each replay over new inputs copied into the captured buffers must equal an
 # eager call on the same inputs bit for bit. T=16 selects the streaming kernels, T=64 the
