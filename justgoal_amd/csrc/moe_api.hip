@@ -272,6 +272,15 @@ int moe_run_ex(const moe_geometry* geom, const void* logits, const void* bias, c
                              (const float*)s13, r.counts, r.offsets, r.sorted_tok, r.C, T, H, I,
                              El, Np, rows_hint, pairs_hint, stream));
   JG_TRY(mark_stage(3, stream));
+  const hipError_t token = jgmoe::launch_gemm2_token(
+      r.C, (const uint8_t*)w2, (const float*)s2, r.counts, r.offsets, r.topk_w, r.pair_of, T,
+      geom->top_k, H, I, El, Np, pairs_hint, (uint16_t*)out, stream);
+  if (token != hipErrorNotSupported) {
+    JG_TRY(token);
+    JG_TRY(mark_stage(4, stream));  // the combine stage is empty
+    JG_TRY(mark_stage(5, stream));
+    return MOE_OK;
+  }
   JG_TRY(jgmoe::launch_gemm2(r.C, (const uint8_t*)w2, (const float*)s2, r.counts, r.offsets,
                              r.sorted_w, jgmoe::Gemm2Out{r.pair_dst, (uint16_t*)out, r.partial},
                              H, I, El, Np, rows_hint, stream));

@@ -67,6 +67,13 @@ hipError_t launch_gemm2_stream(const uint16_t* C, const uint8_t* w2, const float
                                const float* sorted_w, Gemm2Out dst, int H, int I, int E_l,
                                int max_pairs, int mt, hipStream_t stream);
 
+// GEMM2 and combine in one launch for a few tokens: writes every row of out. hipErrorNotSupported
+// where launch_gemm2 and launch_combine serve better, and for I other than 1024, 1536 or 2048.
+hipError_t launch_gemm2_token(const uint16_t* C, const uint8_t* w2, const float* s2,
+                              const int32_t* counts, const int32_t* offsets, const float* topk_w,
+                              const int32_t* pair_of, int T, int K, int H, int I, int E_l,
+                              int max_pairs, int pairs_hint, uint16_t* out, hipStream_t stream);
+
 // Large-tile variants (BM x BN per workgroup, both operands shared through LDS) for long
 // segments. Return hipErrorNotSupported for shapes they do not tile.
 hipError_t launch_gemm1_big(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,

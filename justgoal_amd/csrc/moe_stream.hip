@@ -463,6 +463,203 @@ __global__ __launch_bounds__(256) void gemm2_stream_kernel(
   vm_wait<0>();
 }
 
+// ---- GEMM2 and combine of a few tokens ----------------------------------------------------------
+//
+// Up to 16 tokens fill one 16-row MFMA tile together, whatever experts they picked. A workgroup
+// owns 16 H columns and goes through all active experts, its four waves each a quarter of K: row r
+// of the tile is token r, whose C row for the expert (if it picked it) is the MFMA operand, so the
+// results add up per token in registers: w * (C W2^T) over the token's experts in ascending order,
+// in fp32 and rounded once. No partial rows and no combine launch. Each wave keeps R experts of N
+// K blocks in flight: weights in an LDS ring of D = R * N blocks, the C fragments beside it in
+// registers. Bound by HBM (the weights of the active experts, once); the launch that it saves is
+// a fixed 2-4 us. Measured, call with GEMM2 and combine in two launches -> here: H 4096, I 1536,
+// 128 experts: 1 token 42.0 -> 39.1 us, 4 tokens 102.0 -> 97.2, 12 tokens 210.9 -> 207.4; DS-V3:
+// 1 token 29.3 -> 27.7, 4 tokens 32.8 -> 31.6. R: three experts of 3 blocks instead of four (which
+// leaves one wave per SIMD) 100.0 -> 97.2 us at 4 tokens; two of 4 blocks instead of three
+// 237.0 -> 234.0 us (H 8192, I 2048, 4 tokens).
+//
+// kTokenRows, kTokenPairs: with as many 16-column workgroups as CUs (H 4096) it wins up to 12
+// tokens (above); at 16 it has 80 experts to go through and the item-balanced kernel is ahead
+// (H 4096, I 1536: 237.8 -> 239.7 us). Where the columns do not divide evenly over the CUs the busiest
+// one sets the time, which the saved launch pays for only while there is little to read: DS-V3
+// (448 workgroups) 5 tokens 33.4 -> 32.3 us, 7 tokens 45.2 -> 45.5, 16 tokens 71.1 -> 72.7; H 6144
+// (384), 16 pairs 81.0 -> 83.8. I = 512 gives a wave one block per expert, too little work beside
+// the search for its rows: 4 tokens 52.8 -> 53.9 us, 16 tokens 93.4 -> 101.2.
+constexpr int kTokenRows = 12;
+constexpr int kTokenPairs = 4;
+
+template <int N, int R>
+__global__ __launch_bounds__(256) void gemm2_token_kernel(
+    const uint16_t* __restrict__ C, const uint8_t* __restrict__ w2, const float* __restrict__ s2,
+    const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
+    const float* __restrict__ topk_w, const int32_t* __restrict__ pair_of, int T, int K, int H,
+    int I, int E_l, int max_pairs, uint16_t* __restrict__ out) {
+  constexpr int D = N * R;
+  constexpr int OPS = 6;  // 4 C loads and 2 weight DMAs per step
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kWavesPerGroup][D][kWBlk];
+  __shared__ __attribute__((aligned(16))) v4f red[kWavesPerGroup][kWave];
+  __shared__ __attribute__((aligned(16))) float scl[kWavesPerGroup][R][kWave];
+
+  const int lane = threadIdx.x & (kWave - 1), w = wave_id();
+  const int r16 = lane & 15, g = lane >> 4;
+  const int NKB = N * kWavesPerGroup, kfirst = w * N;  // this wave's K blocks
+  const int h0 = blockIdx.x * 16;
+  const __amdgpu_buffer_rsrc_t cres = make_rsrc(C, (uint32_t)max_pairs * I * 2);
+  const __amdgpu_buffer_rsrc_t wgtres = make_rsrc(topk_w, (uint32_t)T * K * 4);
+  const __amdgpu_buffer_rsrc_t s2res = make_rsrc(s2, (uint32_t)E_l * (H / kBlock) * NKB * 4);
+  const __amdgpu_buffer_rsrc_t pofres = make_rsrc(pair_of, (uint32_t)T * K * 4);
+  const uint32_t dma0 = wblk_dma_off(lane, 0, I), dma1 = wblk_dma_off(lane, 1, I);
+  const uint32_t rd0 = wblk_read_off(lane, 0), rd1 = wblk_read_off(lane, 1);
+  uint8_t* my_ring = &ring[w][0][0];
+
+  // Lane l holds expert l + 64 j's pair count and segment; active[j] has a bit per lane with pairs.
+  int cnt[4], seg[4];
+  unsigned long long active[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int e = j * kWave + lane;
+    cnt[j] = e < E_l ? counts[e] : 0;
+    seg[j] = e < E_l ? offsets[e] : 0;
+    active[j] = __ballot(cnt[j] > 0);
+  }
+  int pk[kMaxTopK];  // pairs of token r16 and their routing weights
+  float wk[kMaxTopK];
+#pragma unroll
+  for (int k = 0; k < kMaxTopK; ++k) {
+    const uint32_t v = r16 < T && k < K ? 4u * (r16 * K + k) : kNoFetch;
+    pk[k] = (int)buf_load32b(pofres, v, 0) | (v == kNoFetch ? -1 : 0);
+    wk[k] = __uint_as_float(buf_load32b(wgtres, v, 0));
+  }
+
+  int left = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) left += __popcll(active[j]);
+  left = uniform(left);
+
+  struct Rows {
+    float wgt;      // routing weight of row r16's pair
+    uint32_t coff;  // its C row (kNoFetch: none)
+  };
+  // Issue side: the next active expert; past the last one nothing is fetched.
+  const uint8_t* wbase = w2;
+  int seg0 = 0, pairs = 0;
+  auto next_expert = [&](int r) {
+    int e = -1;
+    pairs = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (e < 0 && active[j]) {
+        const int l = __ffsll((long long)active[j]) - 1;
+        active[j] &= active[j] - 1;
+        e = j * kWave + l;
+        pairs = __builtin_amdgcn_readlane(cnt[j], l);
+        seg0 = __builtin_amdgcn_readlane(seg[j], l);
+      }
+    }
+    const int x = e < 0 ? 0 : e;
+    const uint32_t so = (uint32_t)((x * (H / kBlock) + h0 / kBlock) * NKB + kfirst) * 4;
+    dma4(s2res, &scl[w][r][0], pairs > 0 && lane < N ? so + 4u * lane : kNoFetch, 0);
+    wbase = uniform(w2 + (size_t)x * H * I);
+  };
+  auto find_rows = [&]() {
+    Rows x = {0.f, kNoFetch};
+#pragma unroll
+    for (int k = 0; k < kMaxTopK; ++k) {
+      const bool in = (uint32_t)(pk[k] - seg0) < (uint32_t)pairs;
+      x.coff = in ? ((uint32_t)pk[k] * I + 32 * g) * 2 : x.coff;
+      x.wgt = in ? wk[k] : x.wgt;
+    }
+    return x;
+  };
+  uint4 a[D][4];
+  auto issue_rows = [&](int d, const Rows& x) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      a[d][c] = buf_load16(cres, x.coff, 2 * ((kfirst + d % N) * kBlock + 8 * c));
+  };
+  auto issue_weights = [&](int d) {
+    const int kb = kfirst + d % N;
+    const __amdgpu_buffer_rsrc_t wres = make_rsrc(uniform(wbase), (uint32_t)H * I);
+    const uint32_t ws = uniform((uint32_t)h0 * I + (uint32_t)kb * kBlock);
+    uint8_t* slot = my_ring + d * kWBlk;
+    dma16_stream(wres, slot, pairs > 0 ? dma0 : kNoFetch, ws);
+    dma16_stream(wres, slot + 1024, pairs > 0 ? dma1 : kNoFetch, ws);
+  };
+
+  Rows rows[R];
+  int seg_r[R], pairs_r[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {  // all weights first: they need no pair lookup
+    next_expert(r);
+    seg_r[r] = seg0, pairs_r[r] = pairs;
+#pragma unroll
+    for (int i = 0; i < N; ++i) issue_weights(r * N + i);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    seg0 = seg_r[r], pairs = pairs_r[r];
+    rows[r] = find_rows();
+#pragma unroll
+    for (int i = 0; i < N; ++i) issue_rows(r * N + i, rows[r]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  v4f acc = {0.f, 0.f, 0.f, 0.f};
+  for (; left > 0; left -= R) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      vm_wait<vm_depth((D - 1) * OPS)>();
+      float sc = ds_read4f(lds_addr(&scl[w][r][lane]));
+      lds_wait_all();
+      lds_fence(sc);
+      const Rows cur = rows[r];
+      next_expert(r);
+      rows[r] = find_rows();
+      v4f ae = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int d = r * N + i;
+        vm_wait<vm_depth((D - 1) * OPS)>();
+        const uint32_t base = lds_addr(my_ring + d * kWBlk);
+        v4u lo = ds_read16(base + rd0), hi = ds_read16(base + rd1);
+        lds_wait(lo, hi);
+        const uint32_t wv[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        v4f t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          v2bf p0, p1, p2, p3;
+          fp8x4_to_bf16x4((int)wv[2 * c], p0, p1);
+          fp8x4_to_bf16x4((int)wv[2 * c + 1], p2, p3);
+          const v8bf bw = v8bf{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+          t = mfma_bf16_16x16x32(bw, __builtin_bit_cast(v8bf, a[d][c]), t);
+        }
+        const float sw =
+            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), i));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ae[q] = fmaf(t[q], sw, ae[q]);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_rows(d, rows[r]);
+        issue_weights(d);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // (rows without a pair are zero rows of the product: kept out, as 0 x NaN or 0 x inf is NaN)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = cur.coff != kNoFetch ? fmaf(ae[q], cur.wgt, acc[q]) : acc[q];
+    }
+  }
+  red[w][lane] = acc;
+  vm_wait<0>();  // no DMA may still target this workgroup's LDS when it retires
+  __syncthreads();
+  if (w == 0 && r16 < T) {
+    v4f s = red[0][lane];
+#pragma unroll
+    for (int k = 1; k < kWavesPerGroup; ++k) s += red[k][lane];
+    const uint32_t h01 = (uint32_t)float_to_bf16_bits(s[0]) | ((uint32_t)float_to_bf16_bits(s[1]) << 16);
+    const uint32_t h23 = (uint32_t)float_to_bf16_bits(s[2]) | ((uint32_t)float_to_bf16_bits(s[3]) << 16);
+    *(uint2*)(out + (size_t)r16 * H + h0 + 4 * g) = uint2{h01, h23};
+  }
+}
+
 }  // namespace
 
 // Persistent grid: `per_cu` workgroups per CU, capped by the largest possible item count.
@@ -578,6 +775,27 @@ hipError_t launch_gemm2_stream(const uint16_t* C, const uint8_t* w2, const float
   if (d == 2) JG_G2S(4, 2)
   JG_G2S(4, 1)
 #undef JG_G2S
+}
+
+hipError_t launch_gemm2_token(const uint16_t* C, const uint8_t* w2, const float* s2,
+                              const int32_t* counts, const int32_t* offsets, const float* topk_w,
+                              const int32_t* pair_of, int T, int K, int H, int I, int E_l,
+                              int max_pairs, int pairs_hint, uint16_t* out, hipStream_t stream) {
+  const int cus = device_cu_count(), groups = H / 16;
+  const bool even = groups <= cus && groups * 8 >= cus * 7;
+  if (T > kTokenRows || (!even && pairs_hint > kTokenPairs) || E_l > 4 * kWave)
+    return hipErrorNotSupported;
+#define JG_G2T(N, R)                                                                            \
+  if (I == N * kWavesPerGroup * kBlock) {                                                       \
+    gemm2_token_kernel<N, R><<<groups, kWavesPerGroup * kWave, 0, stream>>>(                    \
+        C, w2, s2, counts, offsets, topk_w, pair_of, T, K, H, I, E_l, max_pairs, out);          \
+    return hipGetLastError();                                                                   \
+  }
+  JG_G2T(2, 4)
+  JG_G2T(3, 3)
+  JG_G2T(4, 2)
+#undef JG_G2T
+  return hipErrorNotSupported;
 }
 
 }  // namespace jgmoe

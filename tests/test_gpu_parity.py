@@ -418,6 +418,45 @@ def test_streaming_gemm1_split_over_k(gpu, H, T):
         assert ws["counts"].cpu().tolist() == counts
 
 
+def token_kernel_geom(H, I, E, E_l=None):
+    return Geometry(H, I, E, E_l or E, 8, 1, 1, ROUTING_SOFTMAX, f"token-h{H}-i{I}-e{E}")
+
+
+@pytest.mark.parametrize("geom,T", [
+    (token_kernel_geom(4096, 1024, 64), 1),     # H / 16 = 256 workgroups: up to 12 tokens
+    (token_kernel_geom(4096, 1024, 64), 12),
+    (token_kernel_geom(4096, 1024, 64), 13),    # two launches
+    (token_kernel_geom(4096, 1536, 128), 7),     # experts beyond one wave's lanes
+    (token_kernel_geom(3584, 1536, 64, 8), 12),  # tokens without a local pair, fewer workgroups
+    (token_kernel_geom(4096, 2048, 64), 5),
+    (token_kernel_geom(4096, 512, 64), 5),      # I without the kernel
+    (token_kernel_geom(640, 2048, 64, 8), 4),   # uneven columns: up to 4 expected pairs
+    (token_kernel_geom(640, 1024, 64, 8), 5),
+    (DS_V3, 4), (DS_V3, 5)], ids=lambda v: getattr(v, "name", v))
+def test_gemm2_and_combine_in_one_launch(gpu, geom, T):
+    """Both sides of the batches whose GEMM2 adds up each token's experts itself."""
+    check_case(geom, T, gpu, seed=12, rsf=1.0, bias=geom is DS_V3)
+
+
+@pytest.mark.parametrize("T", [2, 12])
+def test_gemm2_in_one_launch_keeps_nan_to_its_token(gpu, T):
+    """An expert with NaN weight scales reaches only the tokens that picked it."""
+    geom = token_kernel_geom(4096, 1024, 64)
+    dev = to_dev(jin.make_activations(geom, T, seed=13), gpu)
+    w13, s13, w2, s2 = weights_for(geom, gpu)[1]
+    kw = dict(gemm1_weights=w13, gemm1_weights_scale=s13, gemm2_weights=w2, local_expert_offset=0,
+              routed_scaling_factor=1.0, geometry=geom)
+    clean = run(**dev, **kw, gemm2_weights_scale=s2)
+    top = torch.topk(dev["routing_logits"].float(), 8, dim=1).indices
+    bad = int(top[0, 0])
+    s2 = s2.clone()
+    s2[bad] = float("nan")
+    out = run(**dev, **kw, gemm2_weights_scale=s2)
+    hit = (top == bad).any(dim=1)
+    assert out[hit].isnan().all()
+    assert torch.equal(out[~hit], clean[~hit])
+
+
 # H = 4096: a row pitch of 4 KiB, where GEMM1's tiles rotate their K order (LDS-tiled at 6 expected
 # rows; 64-row and 128-row large tiles at 16 and 96; 128 rows no longer rotate)
 @pytest.mark.parametrize("T", [48, 128, 768, 1024])
