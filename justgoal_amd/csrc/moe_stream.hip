@@ -466,49 +466,64 @@ __global__ __launch_bounds__(256) void gemm2_stream_kernel(
 // ---- GEMM2 and combine of a few tokens ----------------------------------------------------------
 //
 // Up to 16 tokens fill one 16-row MFMA tile together, whatever experts they picked. A workgroup
-// owns 16 H columns and goes through all active experts, its four waves each a quarter of K: row r
-// of the tile is token r, whose C row for the expert (if it picked it) is the MFMA operand, so the
-// results add up per token in registers: w * (C W2^T) over the token's experts in ascending order,
-// in fp32 and rounded once. No partial rows and no combine launch. Each wave keeps R experts of N
-// K blocks in flight: weights in an LDS ring of D = R * N blocks, the C fragments beside it in
-// registers. Bound by HBM (the weights of the active experts, once); the launch that it saves is
-// a fixed 2-4 us. Measured, call with GEMM2 and combine in two launches -> here: H 4096, I 1536,
-// 128 experts: 1 token 42.0 -> 39.1 us, 4 tokens 102.0 -> 97.2, 12 tokens 210.9 -> 207.4; DS-V3:
-// 1 token 29.3 -> 27.7, 4 tokens 32.8 -> 31.6. R: three experts of 3 blocks instead of four (which
-// leaves one wave per SIMD) 100.0 -> 97.2 us at 4 tokens; two of 4 blocks instead of three
-// 237.0 -> 234.0 us (H 8192, I 2048, 4 tokens).
+// owns `cols` H columns (NB blocks of 16, the last one filled in part) and goes through all active
+// experts, its four waves each a quarter of K: row r of the tile is token r, whose C row for the
+// expert (if it picked it) is the MFMA operand, so the results add up per token in registers:
+// w * (C W2^T) over the token's experts in ascending order, in fp32 and rounded once. No partial
+// rows and no combine launch. Each wave keeps R experts of N K blocks in flight: weights in an LDS
+// ring of D = R * N slots, the C fragments beside it in registers.
+// Bound by HBM (the weights of the active experts, once); the launch that it saves is a fixed 2-4
+// us. `cols` gives every CU one workgroup with an equal share of the columns: with 16 columns per
+// workgroup DS-V3's 448 leave the CUs with one or two each, and the busiest one sets the time (16
+// tokens 72.7 us, with 28 columns 67.1). R: three experts of 3 blocks instead of four 100.0 -> 97.2 us
+// (H 4096, I 1536, 4 tokens); two of 4 blocks instead of three 237.0 -> 234.0 us (H 8192, I 2048).
 //
-// kTokenRows, kTokenPairs: with as many 16-column workgroups as CUs (H 4096) it wins up to 12
-// tokens (above); at 16 it has 80 experts to go through and the item-balanced kernel is ahead
-// (H 4096, I 1536: 237.8 -> 239.7 us). Where the columns do not divide evenly over the CUs the busiest
-// one sets the time, which the saved launch pays for only while there is little to read: DS-V3
-// (448 workgroups) 5 tokens 33.4 -> 32.3 us, 7 tokens 45.2 -> 45.5, 16 tokens 71.1 -> 72.7; H 6144
-// (384), 16 pairs 81.0 -> 83.8. I = 512 gives a wave one block per expert, too little work beside
-// the search for its rows: 4 tokens 52.8 -> 53.9 us, 16 tokens 93.4 -> 101.2.
-constexpr int kTokenRows = 12;
-constexpr int kTokenPairs = 4;
+// Where it is used: up to kTokenRows tokens and kTokenPairs expected pairs. Measured, call with
+// GEMM2 and combine in two launches -> here:
+//   DS-V3: 1 token 29.2 -> 26.4 us, 4 tokens 32.8 -> 30.6, 7 tokens 45.0 -> 43.3, 16 tokens
+//   70.5 -> 67.1; H 4096, I 1536, 128 experts: 1 token 42.0 -> 39.1, 4 tokens 102.0 -> 97.2, 12 tokens
+//   (96 pairs) 210.9 -> 207.4, but 16 tokens (128 pairs, 80 experts one after another) 237.8 -> 239.7;
+//   H 6144, I 1536: 16 pairs 80.4 -> 76.7, 64 pairs 222.2 -> 218.1; H 8192, I 2048, 64 pairs
+//   386.3 -> 375.3.
+// From kTokenCols columns: narrower shares (H 2048: 8 columns) put the same search for an expert's
+// rows on half the weights: H 2048, I 1024, 32 pairs 48.5 -> 52.1 us. The same for one K block per
+// wave (I 512, H 4096): 4 tokens 52.8 -> 53.9 us, 16 tokens 93.4 -> 101.2.
+constexpr int kTokenRows = 16;
+constexpr int kTokenPairs = 96;
+constexpr int kTokenCols = 16;
 
-template <int N, int R>
+template <int NB, int N, int R>
 __global__ __launch_bounds__(256) void gemm2_token_kernel(
     const uint16_t* __restrict__ C, const uint8_t* __restrict__ w2, const float* __restrict__ s2,
     const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
     const float* __restrict__ topk_w, const int32_t* __restrict__ pair_of, int T, int K, int H,
-    int I, int E_l, int max_pairs, uint16_t* __restrict__ out) {
+    int I, int E_l, int max_pairs, int cols, uint16_t* __restrict__ out) {
   constexpr int D = N * R;
-  constexpr int OPS = 6;  // 4 C loads and 2 weight DMAs per step
-  __shared__ __attribute__((aligned(16))) uint8_t ring[kWavesPerGroup][D][kWBlk];
-  __shared__ __attribute__((aligned(16))) v4f red[kWavesPerGroup][kWave];
+  constexpr int OPS = 4 + 2 * NB;  // C loads and weight DMAs per step
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kWavesPerGroup][D][NB * kWBlk];
+  __shared__ __attribute__((aligned(16))) v4f red[kWavesPerGroup][NB][kWave];
   __shared__ __attribute__((aligned(16))) float scl[kWavesPerGroup][R][kWave];
 
   const int lane = threadIdx.x & (kWave - 1), w = wave_id();
   const int r16 = lane & 15, g = lane >> 4;
   const int NKB = N * kWavesPerGroup, kfirst = w * N;  // this wave's K blocks
-  const int h0 = blockIdx.x * 16;
+  const int h0 = blockIdx.x * cols;
+  const int hend = min(h0 + cols, H);
   const __amdgpu_buffer_rsrc_t cres = make_rsrc(C, (uint32_t)max_pairs * I * 2);
   const __amdgpu_buffer_rsrc_t wgtres = make_rsrc(topk_w, (uint32_t)T * K * 4);
   const __amdgpu_buffer_rsrc_t s2res = make_rsrc(s2, (uint32_t)E_l * (H / kBlock) * NKB * 4);
   const __amdgpu_buffer_rsrc_t pofres = make_rsrc(pair_of, (uint32_t)T * K * 4);
-  const uint32_t dma0 = wblk_dma_off(lane, 0, I), dma1 = wblk_dma_off(lane, 1, I);
+  uint32_t dma[NB][2];  // rows past this workgroup's columns are not fetched
+  int sidx[NB];         // scl index of the first K block's scale for this lane's four columns
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int row = 16 * b + 8 * h + (lane >> 3);
+      dma[b][h] = h0 + row < hend ? (uint32_t)(16 * b) * I + wblk_dma_off(lane, h, I) : kNoFetch;
+    }
+    sidx[b] = min((h0 + 16 * b + 4 * g) / kBlock - h0 / kBlock, 1) * N;
+  }
   const uint32_t rd0 = wblk_read_off(lane, 0), rd1 = wblk_read_off(lane, 1);
   uint8_t* my_ring = &ring[w][0][0];
 
@@ -557,8 +572,10 @@ __global__ __launch_bounds__(256) void gemm2_token_kernel(
       }
     }
     const int x = e < 0 ? 0 : e;
-    const uint32_t so = (uint32_t)((x * (H / kBlock) + h0 / kBlock) * NKB + kfirst) * 4;
-    dma4(s2res, &scl[w][r][0], pairs > 0 && lane < N ? so + 4u * lane : kNoFetch, 0);
+    const int hb = h0 / kBlock + (lane >= N);
+    const uint32_t so = (uint32_t)((x * (H / kBlock) + hb) * NKB + kfirst + lane - (lane >= N) * N);
+    dma4(s2res, &scl[w][r][0],
+         pairs > 0 && lane < 2 * N && hb < H / kBlock ? 4u * so : kNoFetch, 0);
     wbase = uniform(w2 + (size_t)x * H * I);
   };
   auto find_rows = [&]() {
@@ -581,9 +598,12 @@ __global__ __launch_bounds__(256) void gemm2_token_kernel(
     const int kb = kfirst + d % N;
     const __amdgpu_buffer_rsrc_t wres = make_rsrc(uniform(wbase), (uint32_t)H * I);
     const uint32_t ws = uniform((uint32_t)h0 * I + (uint32_t)kb * kBlock);
-    uint8_t* slot = my_ring + d * kWBlk;
-    dma16_stream(wres, slot, pairs > 0 ? dma0 : kNoFetch, ws);
-    dma16_stream(wres, slot + 1024, pairs > 0 ? dma1 : kNoFetch, ws);
+    uint8_t* slot = my_ring + d * NB * kWBlk;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      dma16_stream(wres, slot + b * kWBlk, pairs > 0 ? dma[b][0] : kNoFetch, ws);
+      dma16_stream(wres, slot + b * kWBlk + 1024, pairs > 0 ? dma[b][1] : kNoFetch, ws);
+    }
   };
 
   Rows rows[R];
@@ -604,39 +624,51 @@ __global__ __launch_bounds__(256) void gemm2_token_kernel(
     for (int i = 0; i < N; ++i) issue_rows(r * N + i, rows[r]);
   }
   __builtin_amdgcn_sched_barrier(0);
-  v4f acc = {0.f, 0.f, 0.f, 0.f};
+  v4f acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) acc[b] = v4f{0.f, 0.f, 0.f, 0.f};
   for (; left > 0; left -= R) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       vm_wait<vm_depth((D - 1) * OPS)>();
-      float sc = ds_read4f(lds_addr(&scl[w][r][lane]));
+      float sc[NB][N];
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < N; ++i) sc[b][i] = ds_read4f(lds_addr(&scl[w][r][sidx[b] + i]));
       lds_wait_all();
-      lds_fence(sc);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < N; ++i) lds_fence(sc[b][i]);
       const Rows cur = rows[r];
       next_expert(r);
       rows[r] = find_rows();
-      v4f ae = {0.f, 0.f, 0.f, 0.f};
+      v4f ae[NB];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) ae[b] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const int d = r * N + i;
         vm_wait<vm_depth((D - 1) * OPS)>();
-        const uint32_t base = lds_addr(my_ring + d * kWBlk);
-        v4u lo = ds_read16(base + rd0), hi = ds_read16(base + rd1);
-        lds_wait(lo, hi);
-        const uint32_t wv[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        v4f t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          v2bf p0, p1, p2, p3;
-          fp8x4_to_bf16x4((int)wv[2 * c], p0, p1);
-          fp8x4_to_bf16x4((int)wv[2 * c + 1], p2, p3);
-          const v8bf bw = v8bf{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-          t = mfma_bf16_16x16x32(bw, __builtin_bit_cast(v8bf, a[d][c]), t);
+        for (int b = 0; b < NB; ++b) {
+          const uint32_t base = lds_addr(my_ring + (d * NB + b) * kWBlk);
+          v4u lo = ds_read16(base + rd0), hi = ds_read16(base + rd1);
+          lds_wait(lo, hi);
+          const uint32_t wv[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          v4f t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            v2bf p0, p1, p2, p3;
+            fp8x4_to_bf16x4((int)wv[2 * c], p0, p1);
+            fp8x4_to_bf16x4((int)wv[2 * c + 1], p2, p3);
+            const v8bf bw = v8bf{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+            t = mfma_bf16_16x16x32(bw, __builtin_bit_cast(v8bf, a[d][c]), t);
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) ae[b][q] = fmaf(t[q], sc[b][i], ae[b][q]);
         }
-        const float sw =
-            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), i));
-#pragma unroll
-        for (int q = 0; q < 4; ++q) ae[q] = fmaf(t[q], sw, ae[q]);
         __builtin_amdgcn_sched_barrier(0);
         issue_rows(d, rows[r]);
         issue_weights(d);
@@ -644,19 +676,23 @@ __global__ __launch_bounds__(256) void gemm2_token_kernel(
       }
       // (rows without a pair are zero rows of the product: kept out, as 0 x NaN or 0 x inf is NaN)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = cur.coff != kNoFetch ? fmaf(ae[q], cur.wgt, acc[q]) : acc[q];
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          acc[b][q] = cur.coff != kNoFetch ? fmaf(ae[b][q], cur.wgt, acc[b][q]) : acc[b][q];
     }
   }
-  red[w][lane] = acc;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) red[w][b][lane] = acc[b];
   vm_wait<0>();  // no DMA may still target this workgroup's LDS when it retires
   __syncthreads();
-  if (w == 0 && r16 < T) {
-    v4f s = red[0][lane];
+  if (w < NB && r16 < T && h0 + 16 * w + 4 * g < hend) {
+    v4f s = red[0][w][lane];
 #pragma unroll
-    for (int k = 1; k < kWavesPerGroup; ++k) s += red[k][lane];
+    for (int k = 1; k < kWavesPerGroup; ++k) s += red[k][w][lane];
     const uint32_t h01 = (uint32_t)float_to_bf16_bits(s[0]) | ((uint32_t)float_to_bf16_bits(s[1]) << 16);
     const uint32_t h23 = (uint32_t)float_to_bf16_bits(s[2]) | ((uint32_t)float_to_bf16_bits(s[3]) << 16);
-    *(uint2*)(out + (size_t)r16 * H + h0 + 4 * g) = uint2{h01, h23};
+    *(uint2*)(out + (size_t)r16 * H + h0 + 16 * w + 4 * g) = uint2{h01, h23};
   }
 }
 
@@ -781,19 +817,22 @@ hipError_t launch_gemm2_token(const uint16_t* C, const uint8_t* w2, const float*
                               const int32_t* counts, const int32_t* offsets, const float* topk_w,
                               const int32_t* pair_of, int T, int K, int H, int I, int E_l,
                               int max_pairs, int pairs_hint, uint16_t* out, hipStream_t stream) {
-  const int cus = device_cu_count(), groups = H / 16;
-  const bool even = groups <= cus && groups * 8 >= cus * 7;
-  if (T > kTokenRows || (!even && pairs_hint > kTokenPairs) || E_l > 4 * kWave)
+  const int cus = device_cu_count();
+  const int cols = (H + 4 * cus - 1) / (4 * cus) * 4;
+  if (T > kTokenRows || pairs_hint > kTokenPairs || cols < kTokenCols || E_l > 4 * kWave)
     return hipErrorNotSupported;
-#define JG_G2T(N, R)                                                                            \
-  if (I == N * kWavesPerGroup * kBlock) {                                                       \
-    gemm2_token_kernel<N, R><<<groups, kWavesPerGroup * kWave, 0, stream>>>(                    \
-        C, w2, s2, counts, offsets, topk_w, pair_of, T, K, H, I, E_l, max_pairs, out);          \
+#define JG_G2T(NB, N, R)                                                                        \
+  if (cols <= NB * 16 && I == N * kWavesPerGroup * kBlock) {                                    \
+    gemm2_token_kernel<NB, N, R><<<(H + cols - 1) / cols, kWavesPerGroup * kWave, 0, stream>>>( \
+        C, w2, s2, counts, offsets, topk_w, pair_of, T, K, H, I, E_l, max_pairs, cols, out);    \
     return hipGetLastError();                                                                   \
   }
-  JG_G2T(2, 4)
-  JG_G2T(3, 3)
-  JG_G2T(4, 2)
+  JG_G2T(1, 2, 4)
+  JG_G2T(1, 3, 3)
+  JG_G2T(1, 4, 2)
+  JG_G2T(2, 2, 4)
+  JG_G2T(2, 3, 3)
+  JG_G2T(2, 4, 2)
 #undef JG_G2T
   return hipErrorNotSupported;
 }

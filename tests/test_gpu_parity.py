@@ -423,16 +423,18 @@ def token_kernel_geom(H, I, E, E_l=None):
 
 
 @pytest.mark.parametrize("geom,T", [
-    (token_kernel_geom(4096, 1024, 64), 1),     # H / 16 = 256 workgroups: up to 12 tokens
-    (token_kernel_geom(4096, 1024, 64), 12),
-    (token_kernel_geom(4096, 1024, 64), 13),    # two launches
+    (token_kernel_geom(4096, 1024, 64), 1),      # 16 columns per workgroup
+    (token_kernel_geom(4096, 1024, 64), 12),     # 96 expected pairs, the most
+    (token_kernel_geom(4096, 1024, 64), 13),     # two launches
     (token_kernel_geom(4096, 1536, 128), 7),     # experts beyond one wave's lanes
-    (token_kernel_geom(3584, 1536, 64, 8), 12),  # tokens without a local pair, fewer workgroups
-    (token_kernel_geom(4096, 2048, 64), 5),
-    (token_kernel_geom(4096, 512, 64), 5),      # I without the kernel
-    (token_kernel_geom(640, 2048, 64, 8), 4),   # uneven columns: up to 4 expected pairs
-    (token_kernel_geom(640, 1024, 64, 8), 5),
-    (DS_V3, 4), (DS_V3, 5)], ids=lambda v: getattr(v, "name", v))
+    (token_kernel_geom(3584, 1536, 64, 8), 16),  # fewer workgroups; tokens without a local pair
+    (token_kernel_geom(3584, 1536, 64, 8), 17),
+    (token_kernel_geom(4096, 512, 64), 5),       # I without the kernel
+    (token_kernel_geom(3072, 1024, 64, 8), 4),   # too few columns per workgroup
+    (token_kernel_geom(7040, 1024, 64, 8), 16),  # 28 columns, 12 in the last workgroup
+    (token_kernel_geom(8192, 1536, 64, 8), 9),   # 32 columns
+    (token_kernel_geom(8320, 2048, 64, 8), 9),   # 36: two launches
+    (DS_V3, 5), (DS_V3, 15)], ids=lambda v: getattr(v, "name", v))
 def test_gemm2_and_combine_in_one_launch(gpu, geom, T):
     """Both sides of the batches whose GEMM2 adds up each token's experts itself."""
     check_case(geom, T, gpu, seed=12, rsf=1.0, bias=geom is DS_V3)
