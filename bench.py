@@ -51,6 +51,7 @@ GEMM2_TILE_MAX_ROWS = 7
 # ... and of justgoal_amd/csrc/moe_wide.hip (kBigTileRows, kMinRounds), on 256 CUs
 GEMM2_BIG_TILE_ROWS = 64
 GEMM2_WIDE_MIN_ROUNDS = 5
+GEMM2_TOKEN_MAX_ROWS, GEMM2_TOKEN_MAX_PAIRS, GEMM2_TOKEN_MIN_COLS = 16, 96, 16
 CUS = 256
 
 
@@ -202,7 +203,7 @@ def measure(cfg, weight_sets, steps, warmup, settle_ms, dev, seed=None):
     t_floor_ms = max(flops / (PEAK_FP8_TFLOPS * 1e12), bytes_ / (PEAK_HBM_GBS * 1e9)) * 1e3
     g1 = roofline_block("gemm1_swiglu", gemm1_kernel_name(cfg), st["gemm1_swiglu"], g1_flops,
                         g1_bytes, PEAK_FP8_TFLOPS, cfg.name)
-    g2 = roofline_block("gemm2", gemm2_kernel_name(cfg), st["gemm2"], g2_flops, g2_bytes,
+    g2 = roofline_block("gemm2", gemm2_launch_name(cfg), st["gemm2"], g2_flops, g2_bytes,
                         PEAK_BF16_TFLOPS, cfg.name)
     res = dict(workload=cfg.name, geometry=geom.name, tokens=cfg.tokens, seed=seed,
                ms_per_call=ms, steps=steps, warmup_calls=n_warm, weight_sets=len(calls),
@@ -274,6 +275,19 @@ def gemm2_kernel_name(cfg):
     tiles = g.local_experts * -(-g.hidden // 256)
     wide = rows >= GEMM2_BIG_TILE_ROWS or tiles >= GEMM2_WIDE_MIN_ROUNDS * CUS
     return "gemm2_wide_kernel" if wide else "gemm2_big_kernel"
+
+
+def gemm2_launch_name(cfg):
+    """The kernel of the GEMM2 stage: that of gemm2_kernel_name, except for a few tokens, whose
+    GEMM2 and combine are one launch (GEMM2_TOKEN_MAX_ROWS tokens and GEMM2_TOKEN_MAX_PAIRS expected
+    local pairs at most; the rule of justgoal_amd/csrc/moe_stream.hip). Its combine stage is
+    empty."""
+    g = cfg.geom
+    cols = -(-g.hidden // (4 * CUS)) * 4
+    pairs = cfg.tokens * g.top_k * g.local_experts // g.num_experts
+    few = (cfg.tokens <= GEMM2_TOKEN_MAX_ROWS and pairs <= GEMM2_TOKEN_MAX_PAIRS and
+           GEMM2_TOKEN_MIN_COLS <= cols <= 32 and g.intermediate in (1024, 1536, 2048))
+    return "gemm2_token_kernel" if few else gemm2_kernel_name(cfg)
 
 
 def load_traffic(stage, name):

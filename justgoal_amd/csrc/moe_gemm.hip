@@ -2,6 +2,7 @@
 //
 // The GEMMs themselves live in moe_stream.hip (weight streaming, a few pairs per expert),
 // moe_tile.hip (LDS-tiled), moe_big.hip (large tiles) and moe_wide.hip (GEMM2's 256-column tiles).
+// For a few tokens GEMM2 and the combine are one kernel (gemm2_token_kernel, moe_stream.hip).
 // Their arithmetic is the same:
 // GEMM1 runs one v_mfma_f32_16x16x128_f8f6f4 per 128-wide K scale block and adds its fp32 result
 // times hs_scale[kb, token] * s13[e, n/128, kb] to the accumulator

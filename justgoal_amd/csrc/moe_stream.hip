@@ -27,9 +27,9 @@
 // block to bf16 in registers, runs four bf16 MFMAs per K block over the bf16 C rows, scales by
 // the block's weight scale, and stores bf16 rows times the pair's routing weight at the pair's
 // destination (the output row for a token's first local pair, else one of its partial rows).
+// gemm2_token_kernel (below) is GEMM2 of a few tokens with the combine folded in.
 #include "moe_device.h"
 #include "moe_kernels.h"
-
 
 namespace jgmoe {
 

@@ -85,6 +85,19 @@ def test_gemm2_wide_rule_matches_the_library_source():
     assert names["qwen3_t512"] == "gemm2_wide_kernel" and names["ds_t1024"] == "gemm2_big_kernel"
 
 
+def test_few_token_gemm2_rule_matches_the_library_source():
+    import re
+    from justgoal_amd import inputs as jin
+    src = open(os.path.join(ROOT, "justgoal_amd", "csrc", "moe_stream.hip")).read()
+    rows, pairs, cols = (int(re.search(rf"constexpr int kToken{k} = (\d+);", src).group(1))
+                         for k in ("Rows", "Pairs", "Cols"))
+    assert (bench.GEMM2_TOKEN_MAX_ROWS, bench.GEMM2_TOKEN_MAX_PAIRS,
+            bench.GEMM2_TOKEN_MIN_COLS) == (rows, pairs, cols)
+    names = {n: bench.gemm2_launch_name(c) for n, c in jin.CONFIGS.items()}
+    assert names["ds_t16"] == "gemm2_token_kernel"
+    assert names["ds_t64"] == bench.gemm2_kernel_name(jin.CONFIGS["ds_t64"])
+
+
 def test_gemm2_unit_figures_and_roofline_bound():
     # GEMM2: 2*I*H FLOPs per pair; W2 + S2 per active expert, bf16 C read and one bf16 row
     # written per pair
