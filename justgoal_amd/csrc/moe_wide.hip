@@ -248,8 +248,10 @@ __global__ __launch_bounds__(kWideWaves* kWave) void gemm2_wide_kernel(
       }
   };
   // Completes the reads in flight at the end of a step: the second section's weights, the first
-  // halves of the C fragments and the scale. Needed before any control-flow join but the K loop's
-  // own: the compiler takes the asm reads as complete and may copy their registers there.
+  // halves of the C fragments and the scale. It stands before every branch and loop edge: the
+  // compiler takes the asm reads as complete and may copy their registers there (it did copy swn
+  // at the K loop's edge, ahead of the wait). The next step's first section waits for nothing
+  // else, so the wait costs nothing here.
   auto drain = [&] {
     lds_wait_all();
     fence_raw(1);
@@ -311,16 +313,12 @@ __global__ __launch_bounds__(kWideWaves* kWave) void gemm2_wide_kernel(
     };
 
     // One section: a wave's 64 rows x 32 columns (sub-tile s / 2) x 64 of K (half s % 2).
-    auto section = [&](auto BUSY, auto S, int kbi, int kbn, int d, bool head, int parn) {
+    auto section = [&](auto BUSY, auto S, int kbi, int kbn, int d, int parn) {
       constexpr bool B = decltype(BUSY)::v;
       constexpr int s = decltype(S)::v;
-      if constexpr (B) {
+      if constexpr (B && s > 0) {  // (the first section's fragments: drain)
         lds_wait_all();
         fence_raw((s + 1) & 1);
-        if constexpr (s == 0) {
-          fence_a(0);
-          lds_fence(swn);
-        }
         if constexpr (s == 1) fence_a(1);
       }
       if constexpr (kLanded[s] >= 0) {
@@ -356,14 +354,6 @@ __global__ __launch_bounds__(kWideWaves* kWave) void gemm2_wide_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
       } else {
-        if (head) {
-          if constexpr (s == NSEC - 2) read_raw(Int<0>{});
-          if constexpr (s == NSEC - 1) {
-            read_raw(Int<1>{});
-            read_a(Int<0>{});
-            read_sw(kbn, parn);
-          }
-        }
         issue(S, kbi, d);
       }
     };
@@ -372,31 +362,32 @@ __global__ __launch_bounds__(kWideWaves* kWave) void gemm2_wide_kernel(
 #pragma unroll 1
       for (int part = 0; part < 2; ++part) {
         const int end = part ? NKB : NKB - D;
-        if (part) {
-          // the last D blocks' refills come from the next item
-          if constexpr (decltype(BUSY)::v) drain();
-          enter(nxt, more);
-        }
+        if (part) enter(nxt, more);  // the last D blocks' refills come from the next item
         int kbi = part ? 0 : D;
 #pragma unroll 1
         for (; kb < end; ++kb, ++kbi) {
           const bool last = kb + 1 == NKB;
           const int kbn = last ? 0 : kb + 1, parn = last ? par ^ 1 : par;
-          section(BUSY, Int<0>{}, kbi, kbn, slot, last, parn);
-          section(BUSY, Int<1>{}, kbi, kbn, slot, last, parn);
+          section(BUSY, Int<0>{}, kbi, kbn, slot, parn);
+          section(BUSY, Int<1>{}, kbi, kbn, slot, parn);
           if constexpr (NSEC == 4) {
-            section(BUSY, Int<2>{}, kbi, kbn, slot, last, parn);
-            section(BUSY, Int<3>{}, kbi, kbn, slot, last, parn);
+            section(BUSY, Int<2>{}, kbi, kbn, slot, parn);
+            section(BUSY, Int<3>{}, kbi, kbn, slot, parn);
           }
+          if constexpr (decltype(BUSY)::v) drain();
           slot = slot + 1 == D ? 0 : slot + 1;
         }
       }
-      drain();
     };
     // A wave whose 64 rows of the tile are all padding keeps the barriers and its share of the
-    // DMAs, and reads the next item's head.
+    // DMAs, and then reads the next item's head, whose block is refilled only past the next barrier.
     if (WM > 1 && cur.m0 + wm * 64 >= cur.cnt) {
       k_loop(Int<0>{});
+      read_raw(Int<0>{});
+      read_raw(Int<1>{});
+      read_a(Int<0>{});
+      read_sw(0, par ^ 1);
+      drain();
       fence_raw(0);
       convert(0);
     } else {
