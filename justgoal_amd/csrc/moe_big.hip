@@ -612,9 +612,24 @@ __global__ __launch_bounds__((WM * WN + 1) * kWave) void gemm2_big_kernel(
     read_a(lds_addr(&aring[d][0]), 0, a[0]);
   };
 
+  // The head fragments come from asm LDS reads that the compiler takes as complete at once; where
+  // the two loop forms part and join it may copy them (and did, ahead of the first item), so they
+  // are waited for there.
+  auto fence_head = [&] {
+    lds_wait_all();
+#pragma unroll
+    for (int ns = 0; ns < NS; ++ns) {
+      lds_fence(wq[ns][0]);
+      lds_fence(wq[ns][1]);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) lds_fence(a[0][c]);
+  };
+
   int slot = 0;
   __builtin_amdgcn_s_barrier();  // block 0 has landed
   read_head(0);
+  fence_head();
   for (;;) {
     const int it_nn = it_n + stride;
     meta(it_nn < items ? it_nn : (it_n < items ? it_n : it), nn);
@@ -626,18 +641,6 @@ __global__ __launch_bounds__((WM * WN + 1) * kWave) void gemm2_big_kernel(
     // A wave whose 16*MS rows of the tile are all padding only keeps the workgroup's per-step
     // barriers and reads the next item's head at its last step.
     const bool busy = cur.s.m0 + wm * MS * 16 < cur.s.cnt;
-    // The head fragments come from asm LDS reads that the compiler takes as complete at once;
-    // where the two loop forms join it may copy them, so both forms wait for them first.
-    auto fence_head = [&] {
-      lds_wait_all();
-#pragma unroll
-      for (int ns = 0; ns < NS; ++ns) {
-        lds_fence(wq[ns][0]);
-        lds_fence(wq[ns][1]);
-      }
-#pragma unroll
-      for (int c = 0; c < 4; ++c) lds_fence(a[0][c]);
-    };
     if (!busy) {
       int kb = 0;
       do {

@@ -21,10 +21,11 @@ from justgoal_amd import build
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 pytestmark = pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs llvm-objdump")
 
-# the kernel families walked
+# every kernel family of the library
 FAMILIES = ("route_kernel", "route_permute_kernel", "permute_kernel", "combine_kernel",
             "quant_act_kernel", "gemm1_stream_kernel", "gemm1_tile_kernel", "gemm1_big_kernel",
-            "gemm2_stream_kernel", "gemm2_tile_kernel", "gemm2_token_kernel", "gemm2_wide_kernel")
+            "gemm2_stream_kernel", "gemm2_tile_kernel", "gemm2_token_kernel", "gemm2_wide_kernel",
+            "gemm2_big_kernel")
 
 REGS = re.compile(r"\b([va])(?:(\d+)|\[(\d+):(\d+)\])(?!\w)")
 LINE = re.compile(r"^\s+(\S+)\s*(.*?)\s*// ([0-9A-F]+): [0-9A-F ]+(?:<[^>+]*(?:\+0x([0-9a-f]+))?>)?\s*$")
