@@ -71,6 +71,17 @@ struct G1Item {
   int m0, cnt, seg, c0;
 };
 
+// LDS of a gemm1_stream_kernel workgroup, which sets how many a CU holds: the rings and, with K
+// split, the double-buffered partial sums. (Counted without the latter, five blocks per wave took two
+// workgroups per CU where one fits, and half of the grid started over with empty rings when the
+// other half ended. GEMM1 stage, 128 experts all local, I 1536: H 2560 8 tokens 67.2 -> 64.2 us, 64
+// tokens 159.6 -> 154.6; H 5120 64 tokens 304.1 -> 298.0; H 7680 32 tokens 383.3 -> 379.6. Whole-K
+// items take 69.4, 164.5, 305.1 and 406.6.)
+template <int MT, int D, int KS>
+constexpr int g1_stream_lds() {
+  return kWavesPerGroup * D * 2 * kWBlk + (KS > 1 ? 2 * KS * 2 * MT * kWave * (int)sizeof(v4f) : 0);
+}
+
 template <int MT, int D, int KS>
 __global__ __launch_bounds__(256) void gemm1_stream_kernel(
     const uint8_t* __restrict__ hs, const float* __restrict__ hs_scale,
@@ -84,6 +95,8 @@ __global__ __launch_bounds__(256) void gemm1_stream_kernel(
   __shared__ __attribute__((aligned(16))) uint8_t ring[kWavesPerGroup][D][2 * kWBlk];
   // KS > 1: partial sums of an item, double buffered by item parity
   __shared__ __attribute__((aligned(16))) v4f red[KS > 1 ? 2 : 1][KS > 1 ? KS : 1][2 * MT][kWave];
+  static_assert(sizeof(ring) + (KS > 1 ? sizeof(red) : 0) == g1_stream_lds<MT, D, KS>(),
+                "the launcher sizes the grid by this");
 
   const int lane = threadIdx.x & (kWave - 1), w = wave_id();
   const int r16 = lane & 15, g = lane >> 4;
@@ -710,7 +723,7 @@ static inline long long max_m_tiles(int max_pairs, int bm, int E_l) {
   return (max_pairs + bm - 1) / bm + (E_l < max_pairs ? E_l : max_pairs);
 }
 
-// Workgroups per CU that fit the LDS rings (160 KiB per CU).
+// Workgroups per CU that fit its 160 KiB of LDS.
 static inline int groups_per_cu(int lds_bytes) {
   const int n = (160 * 1024) / lds_bytes;
   return n < 1 ? 1 : n > 8 ? 8 : n;
@@ -750,7 +763,7 @@ hipError_t launch_gemm1_stream(const uint8_t* hs, const float* hs_scale, const u
 #define JG_G1S(MT, D, KS)                                                                      \
   {                                                                                            \
     const long long tiles = max_m_tiles(max_pairs, 16 * MT, E_l) * (I / 16);                   \
-    const int grid = persistent_grid(groups_per_cu(kWavesPerGroup * D * 2 * kWBlk),            \
+    const int grid = persistent_grid(groups_per_cu(g1_stream_lds<MT, D, KS>()),                \
                                      (tiles * KS + kWavesPerGroup - 1) / kWavesPerGroup);       \
     gemm1_stream_kernel<MT, D, KS><<<grid, kWavesPerGroup * kWave, 0, stream>>>(               \
         hs, hs_scale, w13, s13, counts, offsets, sorted_tok, C, T, H, I, E_l);                 \
