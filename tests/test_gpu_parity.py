@@ -440,6 +440,32 @@ def test_gemm2_and_combine_in_one_launch(gpu, geom, T):
     check_case(geom, T, gpu, seed=12, rsf=1.0, bias=geom is DS_V3)
 
 
+# 8 of 64 experts local: GEMM2 and combine in one launch for up to 16 tokens
+FEW_LOCAL = token_kernel_geom(4096, 1024, 64, 8)
+
+
+@pytest.mark.parametrize("geom,T,off", [(FEW_LOCAL, 1, 64), (FEW_LOCAL, 16, 64), (DS_V3, 1, 256)],
+                         ids=lambda v: getattr(v, "name", v))
+def test_gemm2_in_one_launch_without_local_pairs(gpu, geom, T, off):
+    """No expert is local: every row of the caller's output becomes zero."""
+    def runner(inp):
+        out = torch.full((T, geom.hidden), float("nan"), dtype=torch.bfloat16, device=gpu)
+        return run(**inp, output=out, geometry=geom), workspace(geom, T, gpu)
+
+    out, ws = check_case(geom, T, gpu, seed=14, local_offset=off, runner=runner)
+    assert int(ws["offsets"][-1]) == 0
+    assert torch.count_nonzero(out).item() == 0
+
+
+@pytest.mark.parametrize("T", [9, 16])
+def test_gemm2_in_one_launch_all_tokens_on_the_same_experts(gpu, T):
+    """Every token picks the same eight experts, all local: full rows of the tile for each."""
+    lg = torch.randn(T, 64, generator=torch.Generator().manual_seed(15))
+    lg[:, :8] += 20.0
+    _, ws = check_case(FEW_LOCAL, T, gpu, seed=15, logits=lg, bias=False, rsf=1.0)
+    assert ws["counts"].cpu().tolist() == [T] * 8
+
+
 @pytest.mark.parametrize("T", [2, 12])
 def test_gemm2_in_one_launch_keeps_nan_to_its_token(gpu, T):
     """An expert with NaN weight scales reaches only the tokens that picked it."""
@@ -641,9 +667,9 @@ def test_route_in_one_launch_matches_oracle(gpu, geom, T, off):
 
 # The operator captured in a HIP graph (serving loops replay one): the library records no memset
 # or allocation, so each replay over new inputs copied into the captured buffers must equal an
-# eager call on the same inputs bit for bit. T=16 selects the streaming kernels, T=64 the
-# LDS-tiled GEMM1 and the streaming GEMM2 (I = 256 is below the LDS-tiled GEMM2's minimum), T=2048
-# the large tiles (T * top_k / E = 0, 2, 64); mini-softmax (I = 384) T=64 the LDS-tiled GEMM2.
+# eager call on the same inputs bit for bit. Mini-DS T=16 and T=64 (T * top_k / E = 0 and 2) select
+# the streaming GEMMs (I = 256 is below the LDS-tiled GEMM2's minimum), T=2048 (64) the large tiles
+# and the wide GEMM2; mini-softmax (I = 384) T=64 the streaming GEMM1 and the LDS-tiled GEMM2.
 @pytest.mark.parametrize("geom,T", [(MINI_DS, 16), (MINI_DS, 64), (MINI_DS, 2048),
                                     (MINI_SOFTMAX, 64)], ids=lambda v: getattr(v, "name", v))
 def test_graph_replay_matches_eager(gpu, geom, T):
@@ -674,6 +700,48 @@ def test_graph_replay_matches_eager(gpu, geom, T):
         ref = run(**fresh, **kw)
         torch.cuda.synchronize()
         assert torch.equal(got, ref), f"replay with seed {seed} differs from the eager call"
+    del g
+    release_workspaces()
+
+
+@pytest.mark.parametrize("T", [1, 7, 12, 16])
+def test_graph_replay_of_few_tokens(gpu, T):
+    """A captured decode step of a few tokens, whose GEMM2 writes all of the output itself: as the
+    routing changes between the replays, tokens lose and regain their local pairs, and one replay
+    has no local pair at all."""
+    geom = FEW_LOCAL
+    say(f"graph replay: {geom.name} T={T}")
+    w = weights_for(geom, gpu)[1]
+    kw = dict(gemm1_weights=w[0], gemm1_weights_scale=w[1], gemm2_weights=w[2],
+              gemm2_weights_scale=w[3], local_expert_offset=0, routed_scaling_factor=1.0,
+              geometry=geom)
+    inputs = [to_dev(jin.make_activations(geom, T, seed=seed), gpu) for seed in (24, 25, 26, 27, 28)]
+    inputs[1]["routing_logits"][:, :8] += 30.0  # every pair local
+    inputs[2]["routing_logits"][:, :8] -= 30.0  # none
+    static = {k: v.clone() for k, v in inputs[0].items()}
+    out = torch.full((T, geom.hidden), float("nan"), dtype=torch.bfloat16, device=gpu)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        run(**static, **kw, output=out)
+    torch.cuda.current_stream().wait_stream(s)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        run(**static, **kw, output=out)
+    for i, fresh in enumerate(inputs):
+        for k, v in fresh.items():
+            static[k].copy_(v)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        ref = run(**fresh, **kw)
+        torch.cuda.synchronize()
+        assert torch.equal(got, ref), f"replay {i} differs from the eager call"
+        local = int(workspace_views(geom, T, workspace(geom, T, gpu))["offsets"][-1])
+        assert i not in (1, 2) or local == (8 * T if i == 1 else 0)
+        assert i != 2 or torch.count_nonzero(got).item() == 0
     del g
     release_workspaces()
 
