@@ -130,6 +130,10 @@ def kernels(tmp_path_factory):
     return out
 
 
+def test_every_kernel_is_walked(kernels):
+    assert all(re.search(rf"\d({'|'.join(FAMILIES)})[IE]", k) for k in kernels)
+
+
 @pytest.mark.parametrize("name", FAMILIES)
 def test_no_register_is_used_while_its_load_is_in_flight(kernels, name):
     mine = {k: v for k, v in kernels.items() if re.search(rf"\d{name}[IE]", k)}

@@ -101,3 +101,27 @@ def test_persistent_grids_fit_the_chip(plan, lds_bytes):
                 assert grid <= CUS * (LDS_PER_CU // lds_bytes[kernel]), (case, kernel, grid)
                 seen.add(kernel)
     assert {f"gemm1_stream_kernel<1,{d},4>" for d in (4, 5, 6, 7, 8)} <= seen
+
+
+def test_bench_names_the_kernels_that_run(plan):
+    """bench.py names each GEMM's kernel by its own copy of the library's selection rules."""
+    import bench
+    from justgoal_amd import inputs as jin
+    tokens = sorted({c.tokens for c in jin.CONFIGS.values()} | set(range(1, 40)) |
+                    {t + d for t in (64, 95, 127, 128, 159, 160, 255, 256, 511, 512, 703, 704,
+                                     1023, 1024, 2047, 2048) for d in (0, 1)})
+    cases = [(g, T) for g in (DS_V3, QWEN3) for T in tokens]
+    for (g, T), launches in zip(cases, plan(cases)):
+        cfg = jin.Config("", g, T)
+        names = [k.split("<")[0] for k, _, _ in launches if k.startswith("gemm")]
+        assert names == [bench.gemm1_kernel_name(cfg), bench.gemm2_launch_name(cfg)], (g, T)
+
+
+@pytest.mark.parametrize("geom,T,route,gemm2", [
+    (DS_V3, 1, 1, 1), (DS_V3, 12, 1, 1), (DS_V3, 13, 2, 1), (DS_V3, 16, 2, 1), (DS_V3, 17, 2, 2),
+    (QWEN3, 12, 1, 1), (QWEN3, 13, 1, 2), (QWEN3, 16, 1, 2), (QWEN3, 17, 2, 2)])
+def test_few_token_calls_take_fewer_launches(plan, geom, T, route, gemm2):
+    """Launches before GEMM1 (routing and permute) and after it (GEMM2 and combine)."""
+    names = [k for k, _, _ in plan([(geom, T)])[0]]
+    at = [i for i, k in enumerate(names) if k.startswith("gemm1")]
+    assert len(at) == 1 and (at[0], len(names) - at[0] - 1) == (route, gemm2)
