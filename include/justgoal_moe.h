@@ -103,8 +103,9 @@ int moe_run_noalloc(const moe_geometry* geom, const void* logits, const void* bi
                     int T, void* stream);
 
 /*
- * Routing + permute stages only (the first two kernels of moe_run_ex), leaving their outputs in
- * the workspace regions described by moe_workspace_layout. The reference has these as the
+ * Routing + permute stages only (the first kernels of moe_run_ex: one launch up to 12 tokens, with
+ * softmax routing up to 16, and two above), leaving their outputs in the workspace regions
+ * described by moe_workspace_layout. The reference has these as the
  * first kernels of its pipeline (goal_full_shape/opus-4.8/moe_fp8_fwd/MOEDIR/main.py:244-248);
  * exported so their integer outputs can be checked bit-exactly.
  */
@@ -122,7 +123,8 @@ enum {
   MOE_WS_SORTED_W,       /* fp32  [Npmax]     routing weight of each pair */
   MOE_WS_C,              /* bf16  [Npmax, I]  SwiGLU activations */
   MOE_WS_PARTIAL,        /* bf16  [T * (k - 1), H]  weighted GEMM2 rows of each token's 2nd..k-th
-                            local pair (k = min(top_k, E_l)); the 1st goes straight into `out` */
+                            local pair (k = min(top_k, E_l)); the 1st goes straight into `out`.
+                            Not written where GEMM2 of a few tokens includes the combine */
   MOE_WS_CHUNK_COUNTS,   /* int32 [ceil(T/c), E_l] pairs per local expert per c-token group,
                             c = 4 for T <= 2048, else 16 (one row per routing workgroup) */
   MOE_WS_PAIR_DST,       /* int32 [Npmax]     GEMM2 destination of each pair: t (row of out) for
@@ -140,7 +142,10 @@ int moe_workspace_layout(const moe_geometry* geom, int T, int64_t* offsets);
  * t14107/moe_kernel.cu:39-52). With n == MOE_NUM_STAGES + 1, every later moe_run / moe_run_ex
  * records events[0] (hipEvent_t) before its first kernel and events[i] after stage i
  * (1 route, 2 permute, 3 GEMM1+SwiGLU, 4 GEMM2, 5 combine) on the call's stream; n == 0 turns
- * it off. Process-wide and not thread-safe: meant for benchmarks.
+ * it off. A stage whose work an earlier one does is empty: permute where routing and permute are one
+ * launch (moe_route_ex above), combine where GEMM2 of a few tokens (at most 16, with at most 96
+ * expected local pairs) adds up each token's rows itself. Process-wide and not thread-safe: meant
+ * for benchmarks.
  */
 #define MOE_NUM_STAGES 5
 int moe_set_stage_events(void* const* events, int n);

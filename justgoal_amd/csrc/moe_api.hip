@@ -1,6 +1,7 @@
 // C ABI of the MoE operator (include/justgoal_moe.h): argument and geometry validation,
 // workspace carving and the launch sequence route -> permute -> GEMM1+SwiGLU -> GEMM2 -> combine,
-// all on the caller's stream. No host synchronisation, no allocation.
+// all on the caller's stream (for a few tokens the first two and the last two are one launch
+// each). No host synchronisation, no allocation.
 #include <hip/hip_runtime.h>
 
 #include <mutex>

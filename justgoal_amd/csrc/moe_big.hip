@@ -785,7 +785,8 @@ constexpr int kB1Wn = 4;
 constexpr int kB1D = 3;
 // GEMM1 for 16..63 expected rows per expert: 64-row tiles (MS = 2, wave tile 32 rows x 32 C
 // columns; 40 KB of DMA per K step for 4.2 MFLOP per CU against 48 KB in the two 64-row
-// workgroups per CU of the LDS-tiled kernel), results bit-identical. Whole call against the
+// workgroups per CU of the LDS-tiled kernel), results bit-identical except where K is rotated (the
+// N-tiles, whose index sets the rotation, are 64 columns wide there and 128 here). Whole call against the
 // LDS-tiled GEMM1, two weight sets in rotation: DS-V3 T=512 211.3 -> 204.4 us, T=768 237.0 ->
 // 218.8, T=1024 249.8 -> 232.1, T=1536 309.9 -> 285.6, T=1792 343.7 -> 294.9; Qwen3-style T=256
 // 446.4 -> 427.9, T=512 485.5 -> 473.2, T=768 536.5 -> 517.9. Below 16 rows DS-V3 is slower on
@@ -795,7 +796,8 @@ constexpr int kB1TallRows = 64;
 constexpr int kB1ShortMs = 2;
 // 128-row tiles below 160 expected rows: 4 compute waves of 64 rows x 64 C columns (2 x 2; five
 // waves per workgroup, so up to 256 VGPRs each, and a quarter less LDS fragment traffic per K
-// step) instead of 8 of 64 x 32. Bit-identical; GEMM1 stage against the 8-wave form, both on
+// step) instead of 8 of 64 x 32. Bit-identical but for the K rotation, which the 8-wave form never
+// has; GEMM1 stage against the 8-wave form, both without it and on
 // the item order of gemm1_sched: DS-V3 T=2048 146.4 -> 142.0 us, T=3072 185.8 -> 182.9, T=4096
 // 202.9 -> 201.4; Qwen3-style T=1024 321 -> 307 (banded order), T=1536 334.3 -> 325.1, T=2048
 // 382.3 -> 371.0. From 160 rows, where GEMM1 turns MFMA-bound, the 8-wave form, whose two waves

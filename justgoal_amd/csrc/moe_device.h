@@ -431,7 +431,8 @@ __device__ __forceinline__ int map_item(const TileMapLds& tml, int item, int ite
 // later (5 is coprime to every block count this applies to) and wraps around, which spreads them.
 // GEMM1 stage, H = 4096 (Qwen3-style): T=128 282 -> 252 us, T=512 290 -> 266, T=1024 312 -> 289, T=1536
 // 333 -> 297; H = 8192 T=512 526 -> 495. Other pitches gain nothing (2048, 3072, 5120 and 6144:
-// within 1%) or lose where M-tiles share activation rows in L2 (DS-V3's 7168, T=14107: 307 -> 342),
+// within 1%) or lose where M-tiles share activation rows in L2 (DS-V3's 7168, T=14107 with 7130
+// pairs: 307 -> 342),
 // so they keep the plain order.
 constexpr int kRotPitchBlocks = 4096 / kBlock;
 __device__ __forceinline__ int k_rotation(int nt, int nkb) { return (5 * nt) % nkb; }

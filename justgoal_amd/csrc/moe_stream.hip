@@ -749,7 +749,8 @@ constexpr int kG2StreamD = 8;
 // (DS-V3 T=1 call 33.3 -> 31.0 us), and evens out the last round (DS-V3 T=48 90.1 -> 88.1, T=128 126.4
 // -> 125.0). From half to one and a half whole-K items per wave that the chip holds the split only
 // adds its reduction (Qwen3-style T=1 43.9 against 44.6 us, T=2 62.1 against 64.2; DS-V3 T=7 46.6
-// against 47.0), so there K stays whole. `expected` counts items under uniform routing.
+// against 47.0), so there K stays whole. `expected` counts one expert for every expected pair up to
+// all of them: an upper bound, since pairs share experts (7 DS-V3 tokens: 7 expected pairs, 3.6 experts).
 
 hipError_t launch_gemm1_stream(const uint8_t* hs, const float* hs_scale, const uint8_t* w13,
                                const float* s13, const int32_t* counts, const int32_t* offsets,

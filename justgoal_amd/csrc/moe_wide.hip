@@ -1,18 +1,21 @@
 // Wide-tile grouped GEMM2: 256 H columns per tile, eight waves that all fetch and all compute.
 //
 // What bounds it. The bf16 MFMAs of a step (128 x 256 x 128: 2048 cycles per SIMD) share the vector
-// issue port with the e4m3 -> bf16 conversion of W2 and the s2 scale FMAs, and on long segments the
-// chip is power-limited: the skewed T=16384 batch runs at 1.64 GHz, and takes 1494 instead of
-// 2040 us on all-zero data. So the tile is chosen for the fewest instructions and LDS bytes per
-// MFMA. A wave owns 64 rows x 64 columns (BM = 128: 2 x 4 waves), so it converts each W2 fragment
-// once per 64 rows (one conversion per 64 FLOP-equal 32x32x16 MFMA pair, half of a 32-row
-// wave tile), reads 24 KB of fragments per step against 32 KB for the same work in 32 x 64
-// wave tiles, and C is fetched once per 256 columns. With eight waves per CU there are 256
-// VGPRs per wave, which the accumulators (64), both halves of the C fragments (64), the MFMA
-// results awaiting their scale (32) and two sections of weights (raw 16, converted 32) fill.
-// Against the 128 x 128 tiles with a producer wave that it replaced, GEMM2 stage, same process:
-// DS-V3 T=2048 96.6 -> 87.5 us, T=4096 133 -> 113, T=6000 172 -> 145, T=14107 292 -> 262, T=16384
-// skewed 2412 -> 1890; Qwen3-style T=1024 210 -> 190, T=2048 345 -> 280.
+// issue port with the e4m3 -> bf16 conversion of W2 and the s2 scale FMAs (MFMA pipes busy 0.45 of the
+// cycles at DS-V3 T=14107 with 7130 pairs, 0.57 at T=16384 skewed), and on long segments the chip is
+// power-limited: the skewed batch (69290 pairs) runs at 1.76 GHz and takes 1942 us, on all-zero data
+// 1415. So the tile is chosen for the fewest instructions and LDS bytes per MFMA. A wave owns 64 rows x
+// 64 columns (BM = 128: 2 x 4 waves), so it converts each W2 fragment once per 64 rows (one
+// conversion per 64 FLOP-equal 32x32x16 MFMA pair, half of a 32-row wave tile), reads 24 KB of
+// fragments per step against 32 KB for the same work in 32 x 64 wave tiles, and C is fetched once per
+// 256 columns. With eight waves per CU there are 256 VGPRs per wave. The accumulators (64), both
+// halves of the C fragments (64), the MFMA results awaiting their scale (32) and two sections of
+// weights (raw 16, converted 32) take 208 of the 241 used; nothing is spilled.
+// Against the 128 x 128 tiles with a producer wave that it replaced, GEMM2 stage, same process (pairs
+// / active experts of each batch; DS-V3 expects T pairs, and a batch's routing bias decides): DS-V3
+// T=2048 (1028 / 24) 96.6 -> 87.5 us, T=4096 (2084 / 28) 133 -> 113, T=6000 (3021 / 29) 172 -> 145,
+// T=14107 (7130 / 29) 292 -> 262, T=16384 skewed (69290 / 22) 2412 -> 1890; Qwen3-style T=1024 210 ->
+// 190, T=2048 345 -> 280. With the expected pairs: T=4096 (4072 / 28) 187 us, T=14107 (13958 / 28) 450.
 //
 // Pipeline. A K step (one 128-wide scale block) is cut into sections of 64 K values x 32 columns
 // per wave (four for BM = 128, two for BM = 64, whose waves own 32 columns). A section issues its
@@ -438,19 +441,24 @@ __global__ __launch_bounds__(kWideWaves* kWave) void gemm2_wide_kernel(
 // Item order. With a multiple of 8 N-tiles the tile-major round-robin order keeps a W2 panel on one
 // XCD for all of an expert's M-tiles. DS-V3 has 28: there XCD-contiguous bands of 4 M-tiles,
 // N-tile-major inside a band, share W2 panels and C rows in an XCD's L2 instead (GEMM2 T=2048 87.5
-// -> 81.9 us, T=4096 119.6 -> 113.0; T=14107 255.6 -> 259.6, T=16384 skewed 1925 -> 1937; for the
-// Qwen3-style 16 N-tiles round-robin is ahead, T=2048 290 against 300).
+// -> 81.9 us, T=4096 119.6 -> 113.0; T=14107 255.6 -> 259.6, T=16384 skewed 1925 -> 1937: the batches
+// above; with the expected pairs T=2048 127.1 -> 126.7, T=3072 159.5 -> 152.9, T=4096 193.7 -> 186.9, T=6000
+// 244.5 -> 236.2, T=14107 445.2 -> 450.3; the skewed call 4192 -> 4164, whose GEMM1 gains. For the
+// Qwen3-style 16 N-tiles round-robin is ahead at T=2048, 312 against 320, level at T=1024, and behind
+// at T=1536, 228 against 219).
 constexpr int kXcds = 8;
 constexpr int kSchedBands = 1 | (4 << 1);
 // Below 144 expected rows most experts have one M-tile, so each W2 byte is read once: the
-// non-temporal hint then keeps GEMM2's rows in the memory-side cache for the combine (whole call,
-// DS-V3 T=2048 249 -> 241 us, T=3072 287.5 -> 280.8, Qwen3-style T=1536 588 -> 583; level at T=4096
-// and T=4900; T=6000 and above are slower with it).
+// non-temporal hint then keeps GEMM2's rows in the memory-side cache for the combine. Whole call
+// without -> with it: DS-V3 T=3072 (1545 pairs) 285.2 -> 280.1 us, T=4096 (2084) 344.8 -> 341.3, Qwen3-style
+// T=1536 553.4 -> 546.2; T=2048 level. Where half of the experts have a second M-tile it costs:
+// DS-V3 T=4096 (4072 pairs) 460.5 -> 464.2, Qwen3-style T=2048 (128 rows, all even) 703.7 -> 722.6; and at
+// T=14107 (13958) 1016 -> 1023, T=16384 skewed 4164 -> 4326.
 constexpr int kSharedRows = 144;
 // 64-row tiles with three slots (two steps, 64 KB of W2, in flight per CU) up to 43 expected rows,
 // if the experts' tiles fill the chip at least five times over: with fewer rounds the
 // 64 x 128 tiles of moe_big.hip lose less in the last one. Qwen3-style (2048 tiles, eight
-// rounds), whole call: T=256 441.8 -> 433.0 us, T=512 476.2 -> 462.2, T=640 487.8 -> 472.8; T=768 (48
+// rounds), whole call (DS-V3: batches of about half the expected pairs): T=256 441.8 -> 433.0 us, T=512 476.2 -> 462.2, T=640 487.8 -> 472.8; T=768 (48
 // rows) 522.3 -> 508.8, but 502.9 with the 128-row tiles. DS-V3 (896 tiles, 3.5 rounds): T=256 164.7
 // against 172.4, T=512 186.5 against 193.4, T=1024 203.6 against 205.4, T=1792 236.6 against 239.0.
 constexpr int kShortRows = 44;
