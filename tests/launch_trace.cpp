@@ -1,6 +1,6 @@
-// Stands in for the HIP runtime (LD_PRELOAD) so that the library's host code runs without a GPU:
-// every launch is written to stdout as "kernel-symbol grid block" instead of reaching a device.
-// The device it reports is a gfx950 with 256 compute units.
+// Stands in for the HIP runtime (loaded ahead of it, with global symbols) so that the library's host
+// code runs without a GPU: every launch is written to stdout as "kernel-symbol grid block" instead
+// of reaching a device. The device it reports is a gfx950 with 256 compute units.
 #define __HIP_PLATFORM_AMD__
 #include <hip/hip_runtime_api.h>
 

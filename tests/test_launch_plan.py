@@ -22,7 +22,8 @@ pytestmark = pytest.mark.skipif(not (shutil.which("g++") and os.path.exists(f"{L
 # Calls moe_run_ex once per line of stdin: the eight geometry fields and T.
 DRIVER = """
 import ctypes, sys
-L = ctypes.CDLL(sys.argv[1])
+ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)  # ahead of the runtime that the library is linked to
+L = ctypes.CDLL(sys.argv[2])
 P = ctypes.c_void_p
 L.moe_run_ex.argtypes = [P] * 9 + [ctypes.c_int, ctypes.c_float, P, P, ctypes.c_int, P]
 p = P(4096)
@@ -55,8 +56,8 @@ def plan(tmp_path_factory):
             " ".join(map(str, (g.hidden, g.intermediate, g.num_experts, g.local_experts, g.top_k,
                                g.n_group, g.topk_group, g.routing_method, T))) + "\n"
             for g, T in cases)
-        out = subprocess.run([sys.executable, "-c", DRIVER, build.LIB_PATH], input=lines, text=True,
-                             capture_output=True, env=dict(os.environ, LD_PRELOAD=str(trace)))
+        out = subprocess.run([sys.executable, "-c", DRIVER, str(trace), build.LIB_PATH], input=lines,
+                             text=True, capture_output=True)
         assert out.returncode == 0, out.stderr
         calls = [c.strip().splitlines() for c in out.stdout.split("#")[1:]]
         assert len(calls) == len(cases)
