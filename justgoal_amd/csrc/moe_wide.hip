@@ -457,10 +457,11 @@ constexpr int kSchedBands = 1 | (4 << 1);
 constexpr int kSharedRows = 144;
 // 64-row tiles with three slots (two steps, 64 KB of W2, in flight per CU) up to 43 expected rows,
 // if the experts' tiles fill the chip at least five times over: with fewer rounds the
-// 64 x 128 tiles of moe_big.hip lose less in the last one. Qwen3-style (2048 tiles, eight
-// rounds), whole call (DS-V3: batches of about half the expected pairs): T=256 441.8 -> 433.0 us, T=512 476.2 -> 462.2, T=640 487.8 -> 472.8; T=768 (48
-// rows) 522.3 -> 508.8, but 502.9 with the 128-row tiles. DS-V3 (896 tiles, 3.5 rounds): T=256 164.7
-// against 172.4, T=512 186.5 against 193.4, T=1024 203.6 against 205.4, T=1792 236.6 against 239.0.
+// 64 x 128 tiles of moe_big.hip lose less in the last one. Whole call, Qwen3-style (2048 tiles, eight
+// rounds): T=256 441.8 -> 433.0 us, T=512 476.2 -> 462.2, T=640 487.8 -> 472.8; T=768 (48 rows) 522.3 ->
+// 508.8, but 502.9 with the 128-row tiles. DS-V3 (896 tiles, 3.5 rounds; batches of about half the
+// expected pairs): T=256 164.7 against 172.4, T=512 186.5 against 193.4, T=1024 203.6 against 205.4,
+// T=1792 236.6 against 239.0.
 constexpr int kShortRows = 44;
 constexpr int kBigTileRows = 64;
 constexpr int kMinRounds = 5;
